@@ -139,6 +139,10 @@ _SIGNATURES = {
     "v1_decode_attention_slots": (_c_i32, [_vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _c_i64,
                                            _c_i32, _vp, _c_i64, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_i32, _c_i32,
                                            _c_i32, ctypes.c_float, _vp]),
+    "v1_decode_attention_slots_ws": (_c_i32, [_vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _vp, _c_i64, _c_i64, _c_i64,
+                                              _c_i32, _vp, _c_i64, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_i32, _c_i32,
+                                              _c_i32, ctypes.c_float, _vp, _c_i64, _vp]),
+    "v1_decode_attention_slots_workspace": (_c_i64, [_c_i32, _c_i32, _c_i32]),
     "v1_union_spans": (_c_i32, [_vp, _vp, _vp, _vp, _c_i32, _c_i32, _c_i32, _vp]),
     "v1_union_normalize_split": (_c_i32, [_vp, _c_i64, _c_i32, _vp, _c_i64, _c_i32, _vp, _vp, _vp, _vp, _vp, _c_i64,
                                           _vp, _vp, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _vp]),

@@ -562,6 +562,20 @@ int v1_decode_attention_slots(const void* q, int64_t q_batch, int64_t q_head, co
                               int64_t req_len, const int32_t* ids, int64_t ids_stride, void* out,
                               int64_t o_batch, int64_t o_head, int32_t rows, int32_t heads_q, int32_t keys,
                               float scale, void* stream);
+
+/* v1_decode_attention_slots with a workspace of
+ * v1_decode_attention_slots_workspace bytes (0: the call needs none): the
+ * parts of a row's keys are then spread over the GPU's XCDs and a second
+ * launch adds them, the same sums in the same order.  A smaller or null
+ * workspace runs the one-launch form. */
+int v1_decode_attention_slots_ws(const void* q, int64_t q_batch, int64_t q_head, const void* k_pool,
+                              int64_t k_slot, int64_t k_head, const void* v_pool, int64_t v_slot,
+                              int64_t v_head, int64_t pool_slots, int32_t head, const int32_t* req,
+                              int64_t req_len, const int32_t* ids, int64_t ids_stride, void* out,
+                              int64_t o_batch, int64_t o_head, int32_t rows, int32_t heads_q, int32_t keys,
+                              float scale, void* workspace, int64_t workspace_bytes,
+                              void* stream);
+int64_t v1_decode_attention_slots_workspace(int32_t rows, int32_t heads_q, int32_t keys);
 #ifdef __cplusplus
 }
 #endif

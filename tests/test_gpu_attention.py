@@ -123,3 +123,67 @@ def test_attend_slots_equals_gather_then_attention(heads):
         two = AT.flash_attn_with_kvcache(qs[:, None], kg, vg, causal=False, softmax_scale=0.09)
         one = AT.attend_slots(qs, kp, vp, req, ids, head, softmax_scale=0.09)
         assert torch.equal(one, two)
+
+
+def _slots_without_workspace(q, kp, vp, req, ids, head, scale):
+    """The slot form's one-launch entry (no workspace), through the C ABI."""
+    L = importlib.import_module("10_20_amd._lib")
+    rows, heads, _ = q.shape
+    out = torch.empty((rows, 1, heads, 128), device=DEV, dtype=torch.bfloat16)
+    L.call("v1_decode_attention_slots", q.data_ptr(), q.stride(0), q.stride(1), kp.data_ptr(), kp.stride(0),
+           kp.stride(1), vp.data_ptr(), vp.stride(0), vp.stride(1), kp.shape[0], head, req.data_ptr(), req.numel(),
+           ids.data_ptr(), ids.stride(0), out.data_ptr(), out.stride(0), out.stride(2), rows, heads, ids.shape[1],
+           scale, L.stream_of(q))
+    return out
+
+
+# rows choose the parts of a row's keys (1 at 4100 and 2100, 2 at 1100, ... 16 from 256 down) and the rows of a
+# work-group; keys the edges of 32-key tiles and of parts (parts without a key among them)
+@pytest.mark.parametrize("rows,keys,heads", [(1, 1, 4), (1, 2048, 1), (3, 31, 2), (17, 33, 3), (130, 65, 4),
+                                             (257, 1000, 2), (600, 97, 4), (1100, 64, 1), (2100, 40, 4), (4100, 32, 3)])
+def test_attend_slots_parts_and_tiles(rows, keys, heads):
+    g = torch.Generator(device=DEV).manual_seed(rows + keys)
+    slots = 5000
+    kp = torch.randn((slots, 2, 128), device=DEV, generator=g).to(torch.bfloat16)
+    vp = torch.randn((slots, 2, 128), device=DEV, generator=g).to(torch.bfloat16)
+    req = torch.randperm(slots, device=DEV, generator=g).to(torch.int32)
+    ids = torch.randint(-2, slots, (rows, keys), device=DEV, generator=g, dtype=torch.int32)
+    q = (3 * torch.randn((rows, heads, 128), device=DEV, generator=g)).to(torch.bfloat16)
+    out = AT.attend_slots(q, kp, vp, req, ids, 1, softmax_scale=0.09)
+    assert torch.equal(out, _slots_without_workspace(q, kp, vp, req, ids, 1, 0.09))
+    kg = torch.where(ids[..., None] >= 0, kp[req[ids.clamp_min(0).long()].long(), 1], 0)
+    vg = torch.where(ids[..., None] >= 0, vp[req[ids.clamp_min(0).long()].long(), 1], 0)
+    two = AT.flash_attn_with_kvcache(q[:, None], kg[:, :, None].contiguous(), vg[:, :, None].contiguous(),
+                                     softmax_scale=0.09)
+    assert torch.equal(out, two)
+    s = torch.matmul(q.double(), kg.double().transpose(1, 2).contiguous()) * 0.09
+    p = torch.softmax(s, -1)
+    ref = torch.matmul(p, vg.double())
+    # rounding to bf16 (8 significant bits: half a unit is up to 2^-8 of the value) and fp32 arithmetic: a score is off
+    # by less than 2^-16 of its terms' sum (130 roundings of 2^-24), which moves p v by as much; p v's own sums round
+    # up to 2048 times, against magnitudes at most p |v|
+    terms = torch.matmul(q.double().abs(), kg.double().abs().transpose(1, 2).contiguous()).amax() * 0.09
+    bound = ref.abs() * (2**-8 + 2**-16) + torch.matmul(p, vg.double().abs()) * (2 * terms * 2**-16 + 2**-13)
+    assert ((out[:, 0].double() - ref).abs() <= bound).all()
+
+
+def test_attend_slots_infinite_values():
+    # a weight times an infinite value is infinite, also where its lower bf16 parts are zero (a lone key has weight 1);
+    # a weight of zero (e^-200 underflows) times it is NaN, as is the sum of both signs; -inf scores weigh nothing
+    kp = torch.zeros((8, 1, 128), device=DEV, dtype=torch.bfloat16)
+    vp = torch.ones((8, 1, 128), device=DEV, dtype=torch.bfloat16)
+    vp[1, 0, 5] = math.inf
+    vp[2, 0, 5] = -math.inf
+    vp[2, 0, 9] = math.inf
+    kp[3, 0, 0] = 200.0
+    kp[4, 0, 0] = -math.inf
+    req = torch.arange(8, device=DEV, dtype=torch.int32)
+    q = torch.zeros((5, 1, 128), device=DEV, dtype=torch.bfloat16)
+    q[:, :, 0] = 1.0
+    ids = torch.tensor([[1, 1, 1], [1, 2, 0], [3, 1, 0], [4, 0, 0], [4, 4, 4]], device=DEV, dtype=torch.int32)
+    got = AT.attend_slots(q, kp, vp, req, ids, 0, softmax_scale=1.0)[:, 0, 0].float().cpu().numpy()
+    assert got[0, 5] == math.inf and (np.delete(got[0], 5) == 1).all()
+    assert math.isnan(got[1, 5]) and got[1, 9] == math.inf and got[1, 0] == 1
+    assert math.isnan(got[2, 5]) and got[2, 0] == 1
+    assert (got[3] == 1).all()
+    assert np.isnan(got[4]).all()
