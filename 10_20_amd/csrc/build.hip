@@ -15,13 +15,24 @@
 // u_d = fl(x_d / m), c_d the FP8 key and s its scale.  Center means add the 8
 // members in order, times 1/8.
 //
-// Two forms: per-kernel drop-ins with the reference's launch shapes, and one
-// fused kernel that builds a batch of buckets, one 1024-thread work-group per
-// bucket (thread = position in the bucket's order): the token's FP8 key stays
-// in registers, an argmin winner stages its key in LDS for the lanes that
-// expand the anchor, each group is sorted by a bitonic network over its
-// unique (score, -position) words, and members move through LDS (groups
-// larger than a wave) or lane shuffles.
+// Two forms: per-kernel drop-ins with the reference's launch shapes, and two
+// launches that build a batch of buckets (thread = position in the order):
+// build_top_kernel takes a bucket through the groups of 1024 and 512 with the
+// tokens' FP8 keys in registers, build_quarter_kernel a quarter of it through
+// the groups of 256 to 16 with their unit vectors there.  An argmin winner
+// stages its vector in LDS, each group is sorted by a bitonic network over its
+// unique (score, -position) words, and members move through LDS or lane
+// permutes.
+//
+// Bound by vector issue: 21 dots of 1024 x 128 terms per bucket, each product
+// and each sum rounded on its own (no FMA, no matrix core can follow that
+// order).  A unit component takes 4.5 operations from its FP8 byte, so the
+// lower levels keep the components (128 registers a token, which is why a
+// work-group is a quarter: three share a CU) and a term of a dot costs its
+// product and its sum; the anchor's components come by DPP row broadcast as
+// an operand of the product, from 8 registers a lane.
+#include <type_traits>
+
 #include "common.h"
 
 // No contraction in this file: every product and every sum written here rounds
@@ -79,6 +90,28 @@ __device__ __forceinline__ float unit_div(float x, float m, float r) {
     const float q0 = x * r;
     return __builtin_fmaf(__builtin_fmaf(-q0, m, x), r, q0);
 }
+
+// Where a token's scale s is a power of two (the format's own scales are),
+// x = c s is exact and x / m = c / (m / s), so its components are quotients of
+// 4-bit significands: fl(c / d) = fl(c h + fl(c l)) with h = fl(1 / d) and
+// l = fl((1 - h d) / d), two operations instead of four.  Checked against the
+// division for all 8 significands and all 2^23 significands of d; within the
+// exponents allowed here no step leaves the normal range.  (With l = e h in
+// place of e / d, 9 of the 67 million pairs differ.)
+__device__ __forceinline__ bool short_units(float s) {
+    const uint32_t bits = __float_as_uint(s);
+    return (bits & 0x807fffffu) == 0 && bits >= (127u - 40u) << 23 && bits <= (127u + 40u) << 23;
+}
+
+struct Recip {
+    float h, l;  // of d = m / s
+};
+
+__device__ __forceinline__ Recip unit_recip(float s, float m, float rm) {
+    return {rm * s, (__builtin_fmaf(-rm, m, 1.0f) / m) * s};
+}
+
+__device__ __forceinline__ float unit_short(float c, Recip r) { return __builtin_fmaf(c, r.h, c * r.l); }
 
 __device__ __forceinline__ void load_key(const uint8_t* row, uint32_t (&c)[kWords]) {
     const uint4* src = reinterpret_cast<const uint4*>(row);
@@ -212,38 +245,6 @@ __global__ __launch_bounds__(128) void assemble_kernel(const uint8_t* __restrict
 }
 
 // ------------------------------------------------------------- fused
-constexpr int kLevels = 7;      // groups of 1024, 512, ..., 16
-constexpr int kSlots = 64;      // anchor and stage slots: four per wave
-constexpr int kAncStride = 33;  // float4 per anchor slot, one of padding
-
-// A token's FP8 key, scale and unit divisor, staged for the lanes that expand it.
-struct Stage {
-    uint32_t c[kWords];
-    float s, m;
-    uint32_t pad[2];
-};
-
-struct BuildSmem {
-    union {
-        struct {
-            float4 anc[kSlots][kAncStride];  // anchor unit vectors: one per wave (groups >= 64) or group
-            Stage st[2][kSlots];             // argmin winners of the first and second dot
-        } d;                                 // live from a level's first anchor to its last dot
-        struct {
-            uint2 c[kWords / 2][kTokens];    // keys by position, 8 bytes of every row per plane
-            int32_t tok[kTokens];
-            float s[kTokens];                // scales
-            float m[kTokens];                // unit divisors
-        } x;                                 // live during a block-wide exchange and the final assembly
-    } u1;
-    union {
-        unsigned long long k[2][kTokens];    // sort keys crossing waves, double-buffered
-        Stage st0[kSlots];                   // first members of the next level's groups
-    } u2;
-    unsigned long long amin[2][kSlots];      // group argmin words (groups above one wave)
-};
-static_assert(sizeof(BuildSmem) <= 160 * 1024, "one work-group per CU");
-
 // Orders this wave's LDS accesses across its lanes (a wave's LDS operations
 // complete in order; the wait and the empty barrier keep the compiler from
 // moving accesses across the point).
@@ -275,241 +276,349 @@ __device__ __forceinline__ uint64_t lane_xor64(uint64_t v) {
     return ((uint64_t)lane_xor<J>((uint32_t)(v >> 32)) << 32) | lane_xor<J>((uint32_t)v);
 }
 
+// Lanes (of 64) whose bit J is clear, and those that keep the larger key of
+// the pair (lane, lane ^ J) while runs of S lanes sort in turn down and up.
+constexpr uint64_t lanes_without(int J) {
+    uint64_t m = 0;
+    for (int l = 0; l < kWave; ++l)
+        if ((l & J) == 0) m |= 1ull << l;
+    return m;
+}
+
 // One compare-exchange step of a descending bitonic network over groups of
-// N (i = position in the group, partner i ^ J, merge size S).
-template <int N, int S, int J>
-__device__ __forceinline__ uint64_t bitonic_step(uint64_t key, int32_t p, uint64_t (*buf)[kTokens], int32_t& nb) {
-    uint64_t other;
+// N (i = position in the group, partner i ^ J, merge size S).  Keys of a
+// group are distinct, so one compare decides: keep the partner's key when it
+// is the larger and this position keeps the maximum, or the smaller and it
+// keeps the minimum.  Which positions keep the maximum is a constant lane
+// mask, but for strides and runs of whole waves, where it is one bit of the
+// wave's number: five vector operations a step.
+template <int N, int S, int J, int T>
+__device__ __forceinline__ uint64_t bitonic_step(uint64_t key, int32_t p, int32_t wave, uint64_t (*buf)[T], int32_t& nb) {
+    uint64_t other, keep_max;
     if constexpr (J >= kWave) {
         buf[nb][p] = key;
         __syncthreads();
         other = buf[nb][p ^ J];
         nb ^= 1;
+        const bool low = ((wave * kWave) & J) == 0, down = S == N || ((wave * kWave) & S) == 0;
+        keep_max = low == down ? ~0ull : 0ull;
     } else {
         other = lane_xor64<J>(key);
+        if constexpr (S == N) keep_max = lanes_without(J);
+        else if constexpr (S < kWave) keep_max = ~(lanes_without(J) ^ lanes_without(S));
+        else keep_max = ((wave * kWave) & S) == 0 ? lanes_without(J) : ~lanes_without(J);
     }
-    const int32_t i = p & (N - 1);
-    const bool take_max = ((i & J) == 0) == ((i & S) == 0);
-    // keys of a group are distinct, so one compare decides: keep the partner's
-    // key when it is the larger and this position keeps the maximum, or the
-    // smaller and it keeps the minimum
-    const bool other_gt = other > key;
-    return other_gt == take_max ? other : key;
+    const uint64_t larger = __builtin_amdgcn_ballot_w64(other > key);
+    return __builtin_amdgcn_inverse_ballot_w64(~(larger ^ keep_max)) ? other : key;
 }
 
-template <int N, int S, int J>
-__device__ __forceinline__ uint64_t bitonic_merge(uint64_t key, int32_t p, uint64_t (*buf)[kTokens], int32_t& nb) {
-    key = bitonic_step<N, S, J>(key, p, buf, nb);
-    if constexpr (J > 1) key = bitonic_merge<N, S, J / 2>(key, p, buf, nb);
+template <int N, int S, int J, int T>
+__device__ __forceinline__ uint64_t bitonic_merge(uint64_t key, int32_t p, int32_t wave, uint64_t (*buf)[T], int32_t& nb) {
+    key = bitonic_step<N, S, J>(key, p, wave, buf, nb);
+    if constexpr (J > 1) key = bitonic_merge<N, S, J / 2>(key, p, wave, buf, nb);
     return key;
 }
 
 // Descending sort of every aligned group of N keys (unique); strides of a
 // wave or more exchange through buf (double-buffered, barriers between).
-template <int N, int S = 2>
-__device__ __forceinline__ uint64_t bitonic_sort(uint64_t key, int32_t p, uint64_t (*buf)[kTokens], int32_t& nb) {
-    key = bitonic_merge<N, S, S / 2>(key, p, buf, nb);
-    if constexpr (S < N) key = bitonic_sort<N, S * 2>(key, p, buf, nb);
+template <int N, int S = 2, int T>
+__device__ __forceinline__ uint64_t bitonic_sort(uint64_t key, int32_t p, int32_t wave, uint64_t (*buf)[T], int32_t& nb) {
+    key = bitonic_merge<N, S, S / 2>(key, p, wave, buf, nb);
+    if constexpr (S < N) key = bitonic_sort<N, S * 2>(key, p, wave, buf, nb);
     return key;
 }
 
-// One 1024-thread work-group per bucket; thread = position in the bucket's
-// current order.  Per level (groups of n): three dots against the group's
-// anchors (first member, b = argmin s0, a = argmin sb), score = dot_a - sb,
-// and a stable descending sort of every group by (score, -position).
-// Groups of at most one wave run without block barriers; larger groups
-// reduce their argmin through LDS atomics and exchange members through LDS.
-__global__ __launch_bounds__(kTokens) void build_buckets_kernel(const uint8_t* __restrict__ pool, int64_t pool_pages,
-                                                                const int32_t* __restrict__ tables,
-                                                                const int32_t* __restrict__ starts,
-                                                                int32_t* __restrict__ perm_out,
-                                                                uint8_t* __restrict__ tmp_out,
-                                                                int32_t* __restrict__ map_out,
-                                                                uint8_t* __restrict__ centers_out) {
-    __shared__ BuildSmem sm;
-    const int32_t p = threadIdx.x;
-    const int64_t b = blockIdx.x;
-    const int32_t* table = tables + b * 16;
-    const float* pool_f = reinterpret_cast<const float*>(pool);
-    auto page_of = [&](int32_t t) __attribute__((always_inline)) {
-        int64_t page = table[t / 64];
-        if ((uint64_t)page >= (uint64_t)pool_pages) page = 0;  // ids outside the pool read page 0
-        return page;
-    };
+// Minimum of (ascending score, position) words over the `width` lanes that
+// share a group (16, 32 or 64), in every lane.
+__device__ __forceinline__ uint64_t lanes_min(uint64_t k, int32_t width) {
+    k = umin64(k, lane_xor64<1>(k));
+    k = umin64(k, lane_xor64<2>(k));
+    k = umin64(k, lane_xor64<4>(k));
+    k = umin64(k, lane_xor64<8>(k));
+    if (width > 16) k = umin64(k, lane_xor64<16>(k));
+    if (width > 32) k = umin64(k, lane_xor64<32>(k));
+    return k;
+}
 
-    int32_t tok = p;
+// Component 16 J + I of the anchor that the lanes of a row share: lane I of
+// the row holds it in a[J].
+template <int I>
+__device__ __forceinline__ float row_bcast(float a) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(a), 0x150 + I, 0xF, 0xF, true));
+}
+
+// acc += unit components u0 .. u3 (dims 4 W .. 4 W + 3) times the anchor's.
+template <int W>
+__device__ __forceinline__ void add_terms(Acc4& acc, const float (&a)[8], float u0, float u1, float u2, float u3) {
+    constexpr int I = 4 * (W & 3), J = W >> 2;
+    acc.add(row_bcast<I>(a[J]) * u0, row_bcast<I + 1>(a[J]) * u1, row_bcast<I + 2>(a[J]) * u2,
+            row_bcast<I + 3>(a[J]) * u3);
+    __builtin_amdgcn_sched_barrier(0);  // (products made ahead of their sums would need registers of their own)
+}
+
+// Page of token t of a bucket (ids outside the pool read page 0).
+__device__ __forceinline__ int64_t page_of(const int32_t* table, int32_t t, int64_t pool_pages) {
+    const int64_t page = table[t / 64];
+    return (uint64_t)page < (uint64_t)pool_pages ? page : 0;
+}
+
+// ---- groups of 1024 and 512: one group per work-group, keys in registers
+// A token's FP8 key, scale and unit divisor, staged for the lanes that expand it.
+struct Stage {
     uint32_t c[kWords];
-    float s, m, rm;  // the token's scale, unit divisor and its reciprocal
-    {
-        const int64_t page = page_of(tok);
-        load_key(pool + page * V1_PAGE_BYTES + (tok % 64) * 128, c);
-        s = pool_f[page * kPageWords + kScaleWord + tok % 64];
-        m = unit_norm(c, s);
-        rm = 1.0f / m;
-    }
+    float s, m, rm;
+};
 
-    // slot of position q's group within q's wave (groups of `width` <= 64
-    // lanes): every wave owns slots 4w .. 4w+3 at every level, so levels run
-    // without block barriers never touch another wave's slots
-    auto wslot = [](int32_t q, int32_t width) __attribute__((always_inline)) {
-        return (q >> 6) * 4 + (q & (kWave - 1)) / width;
-    };
+template <int N>
+struct TopSmem {
+    Stage first;                   // the group's first member
+    Stage win[2][N / kWave];       // each wave's argmin of the first and second dot
+    unsigned long long amin[2];    // the group's argmin words
+    uint64_t k[2][N];              // sort keys crossing waves, double-buffered
+    float m[N];                    // unit divisors
+    int32_t tok[N];
+};
+
+template <bool SHORT, int W = 0>
+__device__ __forceinline__ void dot_keys(Acc4& acc, const float (&a)[8], const uint32_t (&c)[kWords], float s, float m,
+                                         float rm, Recip r) {
+    uint32_t cw = c[W];
+    asm volatile("" : "+v"(cw));  // recomputed per dot: kept, the components would need 128 more registers
+    const float2 lo = fp8_pair<false>(cw), hi = fp8_pair<true>(cw);
+    if constexpr (SHORT)
+        add_terms<W>(acc, a, unit_short(lo.x, r), unit_short(lo.y, r), unit_short(hi.x, r), unit_short(hi.y, r));
+    else
+        add_terms<W>(acc, a, unit_div(lo.x * s, m, rm), unit_div(lo.y * s, m, rm), unit_div(hi.x * s, m, rm),
+                     unit_div(hi.y * s, m, rm));
+    if constexpr (W + 1 < kWords) dot_keys<SHORT, W + 1>(acc, a, c, s, m, rm, r);
+}
+
+// Thread = position in the group (the bucket, or a half of it in the order
+// that the launch before left).  Three dots against the group's anchors
+// (first member, b = argmin s0, a = argmin sb), score = dot_a - sb, and a
+// stable descending sort by (score, -position).  Leaves the order in perm and
+// the unit divisors, as float bits, in map.  64 registers: two groups of 1024
+// share a CU, one's sort beside the other's dots.
+template <int N>
+__global__ __launch_bounds__(N, 8) void build_top_kernel(const uint8_t* __restrict__ pool, int64_t pool_pages,
+                                                         const int32_t* __restrict__ tables,
+                                                         int32_t* __restrict__ perm, int32_t* __restrict__ map) {
+    __shared__ TopSmem<N> sm;
+    const int32_t p = threadIdx.x, lane = p & (kWave - 1);
+    const int32_t wave = __builtin_amdgcn_readfirstlane(p / kWave);
+    const int64_t b = blockIdx.x / (kTokens / N), at = (int64_t)blockIdx.x * N + p;
+
+    const int32_t tok = N == kTokens ? p : perm[at];
+    const int64_t page = page_of(tables + b * 16, tok, pool_pages);
+    uint32_t c[kWords];
+    load_key(pool + page * V1_PAGE_BYTES + (tok % 64) * 128, c);
+    // the token's scale, unit divisor and its reciprocal
+    const float s = reinterpret_cast<const float*>(pool)[page * kPageWords + kScaleWord + tok % 64];
+    const float m = N == kTokens ? unit_norm(c, s) : __int_as_float(map[at]);
+    const float rm = 1.0f / m;
+    const Recip r = unit_recip(s, m, rm);
+    const bool all_short = __builtin_amdgcn_ballot_w64(!short_units(s)) == 0;
+
     auto stage_put = [&](Stage& st) __attribute__((always_inline)) {
         uint4* dst = reinterpret_cast<uint4*>(st.c);
 #pragma unroll
         for (int i = 0; i < kWords / 4; ++i) dst[i] = make_uint4(c[4 * i], c[4 * i + 1], c[4 * i + 2], c[4 * i + 3]);
         st.s = s;
         st.m = m;
+        st.rm = rm;
     };
-    // anchor slot `slot` <- unit vector of the staged token; the `width`
-    // lanes sharing the slot expand one or two key words each
-    auto expand = [&](const Stage& st, int32_t slot, int32_t width) __attribute__((always_inline)) {
-        const int32_t j = p & (width - 1);
-        const int32_t per = width >= 32 ? 1 : 32 / width;  // 1 or 2 (width >= 16)
-        if (j * per < kWords) {
-            const float sa = st.s, ma = st.m;
+    // dot with the staged token: lane i of a row expands its dims i, 16 + i, ...
+    auto dot = [&](const Stage& st) __attribute__((always_inline)) {
+        float a[8];
+        const float sa = st.s, ma = st.m, ra = st.rm;
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                if (q < per) {
-                    const int32_t w = j * per + q;
-                    const uint32_t cw = st.c[w];
-                    const float2 lo = fp8_pair<false>(cw), hi = fp8_pair<true>(cw);
-                    sm.u1.d.anc[slot][w] =
-                        make_float4((lo.x * sa) / ma, (lo.y * sa) / ma, (hi.x * sa) / ma, (hi.y * sa) / ma);
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t w = st.c[4 * j + ((lane & 15) >> 2)] >> (8 * (lane & 3));
+            a[j] = unit_div(fp8_at<0>(w) * sa, ma, ra);
+        }
+        Acc4 acc;
+        if (all_short) dot_keys<true>(acc, a, c, s, m, rm, r);
+        else dot_keys<false>(acc, a, c, s, m, rm, r);
+        return acc.total();
+    };
+    // group argmin (leftmost minimum, -0.0 == +0.0): every wave's winner stages
+    // its key; returns the group's winner's wave
+    auto argmin = [&](float v, int32_t i) __attribute__((always_inline)) {
+        const uint64_t k = lanes_min(((uint64_t)score_key(v) << 32) | (uint32_t)p, kWave);
+        if ((uint32_t)k == (uint32_t)p) {
+            stage_put(sm.win[i][wave]);
+            atomicMin(&sm.amin[i], (unsigned long long)k);
+        }
+        __syncthreads();
+        return (int32_t)(uint32_t)sm.amin[i] / kWave;
+    };
+    if (p < 2) sm.amin[p] = ~0ull;
+    if (p == 0) stage_put(sm.first);
+    sm.m[p] = m;
+    sm.tok[p] = tok;
+    __syncthreads();
+
+    const float s0 = dot(sm.first);
+    const float sb = dot(sm.win[0][argmin(s0, 0)]);
+    const float score = dot(sm.win[1][argmin(sb, 1)]) - sb;
+    int32_t nb = 0;
+    const uint64_t key = bitonic_sort<N>(((uint64_t)score_key(score) << 32) | (0xffffffffu - (uint32_t)p), p, wave,
+                                         sm.k, nb);
+    const int32_t from = (int32_t)(0xffffffffu - (uint32_t)key);  // old position of the new member
+    perm[at] = sm.tok[from];
+    map[at] = __float_as_int(sm.m[from]);
+}
+
+// ---- groups of 256 to 16: a quarter of a bucket per work-group
+constexpr int kQuarter = 256;
+constexpr int kQuarterWaves = kQuarter / kWave;
+
+// Tokens are numbered by their first position in the quarter; a thread's
+// token moves as its number.
+struct QuarterSmem {
+    uint4 c[kQuarter][8];             // keys: 16-byte chunk j of token t at j ^ (t % 8)
+    float4 v[kQuarter];               // scale, unit divisor, its reciprocal, token in the bucket (int bits)
+    Recip r[kQuarter];
+    unsigned long long amin[2][2];    // argmin words of the groups above one wave
+    uint64_t k[2][kQuarter];          // sort keys crossing waves, double-buffered
+    int32_t first[kQuarterWaves];     // first token of every wave
+};
+
+template <int W = 0>
+__device__ __forceinline__ void dot_units(Acc4& acc, const float (&a)[8], const float (&u)[128]) {
+    add_terms<W>(acc, a, u[4 * W], u[4 * W + 1], u[4 * W + 2], u[4 * W + 3]);
+    if constexpr (W + 1 < kWords) dot_units<W + 1>(acc, a, u);
+}
+
+// Thread = position in the quarter; the levels as above.  A level makes its
+// token's unit vector from the key in LDS (moving 128 registers instead costs
+// more LDS time than that takes vector time: 740 against XXX us for 2048
+// buckets) and holds it through three dots.  Groups of at most one wave run
+// without barriers.  Then the quarter's pages, member map, order and centers.
+__global__ __launch_bounds__(kQuarter, 3) void build_quarter_kernel(const uint8_t* __restrict__ pool, int64_t pool_pages,
+                                                                    const int32_t* __restrict__ tables,
+                                                                    const int32_t* __restrict__ starts,
+                                                                    int32_t* __restrict__ perm_out,
+                                                                    uint8_t* __restrict__ tmp_out,
+                                                                    int32_t* __restrict__ map_out,
+                                                                    uint8_t* __restrict__ centers_out) {
+    __shared__ QuarterSmem sm;
+    const int32_t p = threadIdx.x, lane = p & (kWave - 1);
+    const int32_t wave = __builtin_amdgcn_readfirstlane(p / kWave);
+    const int64_t b = blockIdx.x / (kTokens / kQuarter);
+    const int32_t at = (int32_t)(blockIdx.x % (kTokens / kQuarter)) * kQuarter + p;  // position in the bucket
+
+    int32_t id = p;
+    bool all_short;
+    {
+        const int32_t tok = perm_out[b * kTokens + at];
+        const float m = __int_as_float(map_out[b * kTokens + at]);
+        const int64_t page = page_of(tables + b * 16, tok, pool_pages);
+        const uint4* src = reinterpret_cast<const uint4*>(pool + page * V1_PAGE_BYTES + (tok % 64) * 128);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sm.c[p][j ^ (p & 7)] = src[j];
+        const float s = reinterpret_cast<const float*>(pool)[page * kPageWords + kScaleWord + tok % 64], rm = 1.0f / m;
+        sm.v[p] = make_float4(s, m, rm, __int_as_float(tok));
+        sm.r[p] = unit_recip(s, m, rm);
+        all_short = __syncthreads_and(short_units(s));
+    }
+    float u[128];  // the token's unit vector
+    auto make_units = [&]() __attribute__((always_inline)) {
+        const float4 v = sm.v[id];
+        const Recip r = sm.r[id];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint4 w4 = sm.c[id][j ^ (id & 7)];
+            const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float2 lo = fp8_pair<false>(words[q]), hi = fp8_pair<true>(words[q]);
+                float* d = u + 16 * j + 4 * q;
+                if (all_short) {
+                    d[0] = unit_short(lo.x, r);
+                    d[1] = unit_short(lo.y, r);
+                    d[2] = unit_short(hi.x, r);
+                    d[3] = unit_short(hi.y, r);
+                } else {
+                    d[0] = unit_div(lo.x * v.x, v.y, v.z);
+                    d[1] = unit_div(lo.y * v.x, v.y, v.z);
+                    d[2] = unit_div(hi.x * v.x, v.y, v.z);
+                    d[3] = unit_div(hi.y * v.x, v.y, v.z);
                 }
             }
         }
     };
-    auto dot = [&](int32_t slot) __attribute__((always_inline)) {
-        // the unit components are recomputed per dot: kept across the three
-        // dots of a level they would need 128 more registers
+    // dot with token t's unit vector: lane i of a row expands its dims i, 16 + i, ...
+    auto dot = [&](int32_t t) __attribute__((always_inline)) {
+        const float4 v = sm.v[t];
+        const uint8_t* row = reinterpret_cast<const uint8_t*>(sm.c[t]) + (lane & 15);
+        float a[8];
 #pragma unroll
-        for (int w = 0; w < kWords; ++w) asm volatile("" : "+v"(c[w]));
-        const float4* a = sm.u1.d.anc[slot];
+        for (int j = 0; j < 8; ++j) a[j] = unit_div(fp8_at<0>(row[16 * (j ^ (t & 7))]) * v.x, v.y, v.z);
         Acc4 acc;
-#pragma unroll 4
-        for (int w = 0; w < kWords; ++w) {
-            const float4 av = a[w];
-            const float2 lo = fp8_pair<false>(c[w]), hi = fp8_pair<true>(c[w]);
-            acc.add((unit_div(lo.x * s, m, rm) * av.x), (unit_div(lo.y * s, m, rm) * av.y),
-                    (unit_div(hi.x * s, m, rm) * av.z), (unit_div(hi.y * s, m, rm) * av.w));
-        }
+        dot_units(acc, a, u);
         return acc.total();
     };
-    // group argmin (leftmost minimum, -0.0 == +0.0): the winner stages its
-    // key in st[m][its slot]; returns the winner's position
-    auto argmin = [&](float v, int32_t n, int32_t width, int32_t m) __attribute__((always_inline)) {
-        uint64_t k = ((uint64_t)score_key(v) << 32) | (uint32_t)p;
-        k = umin64(k, lane_xor64<1>(k));  // width >= 16
-        k = umin64(k, lane_xor64<2>(k));
-        k = umin64(k, lane_xor64<4>(k));
-        k = umin64(k, lane_xor64<8>(k));
-        if (width > 16) k = umin64(k, lane_xor64<16>(k));
-        if (width > 32) k = umin64(k, lane_xor64<32>(k));
-        if ((uint32_t)k == (uint32_t)p) stage_put(sm.u1.d.st[m][wslot(p, width)]);
-        if (n > kWave) {
-            if ((p & (kWave - 1)) == 0) atomicMin(&sm.amin[m][p / n], (unsigned long long)k);
+    // token of the group's minimum (leftmost, -0.0 == +0.0)
+    auto argmin = [&](float v, auto group, int32_t i) __attribute__((always_inline)) {
+        constexpr int32_t n = decltype(group)::value;
+        uint64_t k = lanes_min(((uint64_t)score_key(v) << 32) | (uint32_t)(p << 8 | id), n < kWave ? n : kWave);
+        if constexpr (n > kWave) {
+            if (lane == 0) atomicMin(&sm.amin[i][wave / (n / kWave)], (unsigned long long)k);
             __syncthreads();
-            k = sm.amin[m][p / n];
-        } else {
-            wave_sync();
+            k = sm.amin[i][wave / (n / kWave)];
         }
-        return (int32_t)(uint32_t)k;
+        return (int32_t)(k & 255);
     };
-    if (p < 2 * kSlots) (&sm.amin[0][0])[p] = ~0ull;
-    if (p == 0) stage_put(sm.u2.st0[0]);
+    if (p < 4) (&sm.amin[0][0])[p] = ~0ull;
     __syncthreads();
 
-#pragma unroll 1
-    for (int level = 0; level < kLevels; ++level) {
-        const int32_t n = kTokens >> level;
-        const int32_t width = n < kWave ? n : kWave;
-        const int32_t slot = wslot(p, width);
-        expand(sm.u2.st0[n > kWave ? p / n : slot], slot, width);  // the group's first member
-        wave_sync();
-        const float s0 = dot(slot);
-        const int32_t bpos = argmin(s0, n, width, 0);
-        expand(sm.u1.d.st[0][wslot(bpos, width)], slot, width);
-        wave_sync();
-        const float sb = dot(slot);
-        const int32_t apos = argmin(sb, n, width, 1);
-        expand(sm.u1.d.st[1][wslot(apos, width)], slot, width);
-        wave_sync();
-        const float score = (dot(slot) - sb);
-        uint64_t key = ((uint64_t)score_key(score) << 32) | (0xffffffffu - (uint32_t)p);
-        {
-            auto* kb = reinterpret_cast<uint64_t (*)[kTokens]>(sm.u2.k);
-            int32_t nb = 0;
-            switch (level) {
-                case 0: key = bitonic_sort<1024>(key, p, kb, nb); break;
-                case 1: key = bitonic_sort<512>(key, p, kb, nb); break;
-                case 2: key = bitonic_sort<256>(key, p, kb, nb); break;
-                case 3: key = bitonic_sort<128>(key, p, kb, nb); break;
-                case 4: key = bitonic_sort<64>(key, p, kb, nb); break;
-                case 5: key = bitonic_sort<32>(key, p, kb, nb); break;
-                default: key = bitonic_sort<16>(key, p, kb, nb); break;
-            }
-        }
-        const int32_t from = (int32_t)(0xffffffffu - (uint32_t)key);  // old position of the new member
-        const int32_t half = n >> 1;
-        if (n > kWave) {
-            // every wave is past its last dot (the sort crossed a barrier):
-            // the exchange area may overwrite the anchors
-#pragma unroll
-            for (int w = 0; w < kWords / 2; ++w) sm.u1.x.c[w][p] = make_uint2(c[2 * w], c[2 * w + 1]);
-            sm.u1.x.tok[p] = tok;
-            sm.u1.x.s[p] = s;
-            sm.u1.x.m[p] = m;
+    int32_t first = 0;  // first token of the group
+    auto level = [&](auto group) __attribute__((always_inline)) {
+        constexpr int32_t n = decltype(group)::value, half = n >> 1;
+        make_units();
+        const float s0 = dot(first);
+        const float sb = dot(argmin(s0, group, 0));
+        const float score = dot(argmin(sb, group, 1)) - sb;
+        int32_t nb = 0;
+        const uint64_t key = bitonic_sort<n>(((uint64_t)score_key(score) << 32) | ~(uint32_t)(p << 8 | id), p, wave,
+                                             sm.k, nb);
+        id = (int32_t)(~(uint32_t)key & 255u);
+        if constexpr (half > kWave) {
+            // (the sort's barriers lie between the argmin words' last use and this)
+            if (lane == 0) sm.first[wave] = id;
+            if (p < 4) (&sm.amin[0][0])[p] = ~0ull;
             __syncthreads();
-#pragma unroll
-            for (int w = 0; w < kWords / 2; ++w) {
-                const uint2 v = sm.u1.x.c[w][from];
-                c[2 * w] = v.x;
-                c[2 * w + 1] = v.y;
-            }
-            tok = sm.u1.x.tok[from];
-            s = sm.u1.x.s[from];
-            m = sm.u1.x.m[from];
-            rm = 1.0f / m;
-            if (p < 2 * kSlots) (&sm.amin[0][0])[p] = ~0ull;
-            if (level + 1 < kLevels && (p & (half - 1)) == 0)
-                stage_put(sm.u2.st0[half > kWave ? p / half : wslot(p, half)]);
-            __syncthreads();
-        } else {
-            const int32_t src = from & (kWave - 1);  // same wave
-#pragma unroll
-            for (int w = 0; w < kWords; ++w) c[w] = (uint32_t)__shfl((int)c[w], src, kWave);
-            tok = __shfl(tok, src, kWave);
-            s = __shfl(s, src, kWave);
-            m = __shfl(m, src, kWave);
-            rm = __shfl(rm, src, kWave);
-            if (level + 1 < kLevels && (p & (half - 1)) == 0) stage_put(sm.u2.st0[wslot(p, half)]);
-            wave_sync();
+            first = sm.first[wave & ~(half / kWave - 1)];
+        } else if constexpr (half >= 16) {
+            first = __builtin_amdgcn_ds_bpermute((lane & ~(half - 1)) << 2, id);
         }
-    }
+    };
+    level(std::integral_constant<int32_t, 256>());
+    level(std::integral_constant<int32_t, 128>());
+    level(std::integral_constant<int32_t, 64>());
+    level(std::integral_constant<int32_t, 32>());
+    level(std::integral_constant<int32_t, 16>());
 
     // final order: perm, the assembled pages, member map and centers
-    const int64_t page = page_of(tok);
-    perm_out[b * kTokens + p] = tok;
-    map_out[b * kTokens + p] = starts[b] + tok;
-    uint8_t* tp = tmp_out + (b * 16 + p / 64) * V1_PAGE_BYTES;
-    uint4* row = reinterpret_cast<uint4*>(tp + (p % 64) * 128);
+    const float4 v = sm.v[id];
+    const int32_t tok = __float_as_int(v.w);
+    perm_out[b * kTokens + at] = tok;
+    map_out[b * kTokens + at] = starts[b] + tok;
+    uint8_t* tp = tmp_out + (b * 16 + at / 64) * V1_PAGE_BYTES;
+    uint4* row = reinterpret_cast<uint4*>(tp + (at % 64) * 128);
 #pragma unroll
-    for (int i = 0; i < kWords / 4; ++i) row[i] = make_uint4(c[4 * i], c[4 * i + 1], c[4 * i + 2], c[4 * i + 3]);
-    reinterpret_cast<float*>(tp)[kScaleWord + p % 64] = s;
-    __syncthreads();  // every wave is past its last dot
-#pragma unroll
-    for (int w = 0; w < kWords / 2; ++w) sm.u1.x.c[w][p] = make_uint2(c[2 * w], c[2 * w + 1]);
-    sm.u1.x.s[p] = s;
-    wave_sync();  // a center's 8 members are rows of this wave
-    // center p / 8: lane r of the 8 members computes dims 16r .. 16r+15
-    const int32_t r = p & 7, m0 = p & ~7;
+    for (int j = 0; j < 8; ++j) row[j] = sm.c[id][j ^ (id & 7)];
+    reinterpret_cast<float*>(tp)[kScaleWord + at % 64] = v.x;
+    // center at / 8: lane r of the 8 members computes dims 16r .. 16r+15
+    const int32_t r = p & 7;
     float mean[16];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-        const uint2 w01 = sm.u1.x.c[2 * r][m0 + j], w23 = sm.u1.x.c[2 * r + 1][m0 + j];
-        const float sj = sm.u1.x.s[m0 + j];
-        const uint32_t words[4] = {w01.x, w01.y, w23.x, w23.y};
+        const int32_t t = __builtin_amdgcn_ds_bpermute(((lane & ~7) + j) << 2, id);
+        const uint4 w4 = sm.c[t][r ^ (t & 7)];
+        const float sj = sm.v[t].x;
+        const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const float x0 = (fp8_at<0>(words[q]) * sj), x1 = (fp8_at<1>(words[q]) * sj);
@@ -542,11 +651,12 @@ __global__ __launch_bounds__(kTokens) void build_buckets_kernel(const uint8_t* _
         packed[q] = e4m3_code(mean[4 * q] / scale) | (e4m3_code(mean[4 * q + 1] / scale) << 8) |
                     (e4m3_code(mean[4 * q + 2] / scale) << 16) |
                     (e4m3_code(mean[4 * q + 3] / scale) << 24);
-    const int32_t center = p / 8;
+    const int32_t center = at / 8;
     uint8_t* cp = centers_out + (b * 2 + center / 64) * V1_PAGE_BYTES;
     *reinterpret_cast<uint4*>(cp + (center % 64) * 128 + 16 * r) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
     if (r == 0) reinterpret_cast<float*>(cp)[kScaleWord + center % 64] = scale;
 }
+
 
 }  // namespace
 }  // namespace v1
@@ -602,8 +712,16 @@ extern "C" int v1_build_buckets(const void* pool, int64_t pool_pages, const int3
                    (reinterpret_cast<uintptr_t>(centers) & 15) == 0,
                "build_buckets: pool, tmp and centers must be 16-byte aligned");
     if (buckets == 0) return V1_OK;
-    hipLaunchKernelGGL(build_buckets_kernel, dim3((uint32_t)buckets), dim3(kTokens), 0, as_stream(stream),
-                       static_cast<const uint8_t*>(pool), pool_pages, tables, starts, perm, static_cast<uint8_t*>(tmp), mapping,
-                       static_cast<uint8_t*>(centers));
-    return V1_LAUNCHED("build_buckets");
+    hipLaunchKernelGGL(build_top_kernel<1024>, dim3((uint32_t)buckets), dim3(1024), 0, as_stream(stream),
+                       static_cast<const uint8_t*>(pool), pool_pages, tables, perm, mapping);
+    int rc = V1_LAUNCHED("build_buckets: 1024");
+    if (rc != V1_OK) return rc;
+    hipLaunchKernelGGL(build_top_kernel<512>, dim3((uint32_t)buckets * 2), dim3(512), 0, as_stream(stream),
+                       static_cast<const uint8_t*>(pool), pool_pages, tables, perm, mapping);
+    rc = V1_LAUNCHED("build_buckets: 512");
+    if (rc != V1_OK) return rc;
+    hipLaunchKernelGGL(build_quarter_kernel, dim3((uint32_t)buckets * (kTokens / kQuarter)), dim3(kQuarter), 0,
+                       as_stream(stream), static_cast<const uint8_t*>(pool), pool_pages, tables, starts, perm,
+                       static_cast<uint8_t*>(tmp), mapping, static_cast<uint8_t*>(centers));
+    return V1_LAUNCHED("build_buckets: quarters");
 }
