@@ -30,7 +30,9 @@
 // lower levels keep the components (128 registers a token, which is why a
 // work-group is a quarter: three share a CU) and a term of a dot costs its
 // product and its sum; the anchor's components come by DPP row broadcast as
-// an operand of the product, from 8 registers a lane.
+// an operand of the product, from 8 registers a lane.  2048 buckets take
+// 161 + 131 + 459 us (one launch with every component made anew for every dot
+// 1266), four 24 + 14 + 25 us (155); the vector units issue 94-96% of the time.
 #include <type_traits>
 
 #include "common.h"
@@ -492,8 +494,8 @@ __device__ __forceinline__ void dot_units(Acc4& acc, const float (&a)[8], const 
 
 // Thread = position in the quarter; the levels as above.  A level makes its
 // token's unit vector from the key in LDS (moving 128 registers instead costs
-// more LDS time than that takes vector time: 740 against XXX us for 2048
-// buckets) and holds it through three dots.  Groups of at most one wave run
+// more LDS time than that takes vector time: 740 against 527 us for 2048
+// buckets when both were tried) and holds it through three dots.  Groups of at most one wave run
 // without barriers.  Then the quarter's pages, member map, order and centers.
 __global__ __launch_bounds__(kQuarter, 3) void build_quarter_kernel(const uint8_t* __restrict__ pool, int64_t pool_pages,
                                                                     const int32_t* __restrict__ tables,
@@ -524,37 +526,43 @@ __global__ __launch_bounds__(kQuarter, 3) void build_quarter_kernel(const uint8_
     }
     float u[128];  // the token's unit vector
     auto make_units = [&]() __attribute__((always_inline)) {
-        const float4 v = sm.v[id];
-        const Recip r = sm.r[id];
+        auto each_word = [&](auto unit) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint4 w4 = sm.c[id][j ^ (id & 7)];
-            const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
+            for (int j = 0; j < 8; ++j) {
+                const uint4 w4 = sm.c[id][j ^ (id & 7)];
+                const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float2 lo = fp8_pair<false>(words[q]), hi = fp8_pair<true>(words[q]);
-                float* d = u + 16 * j + 4 * q;
-                if (all_short) {
-                    d[0] = unit_short(lo.x, r);
-                    d[1] = unit_short(lo.y, r);
-                    d[2] = unit_short(hi.x, r);
-                    d[3] = unit_short(hi.y, r);
-                } else {
-                    d[0] = unit_div(lo.x * v.x, v.y, v.z);
-                    d[1] = unit_div(lo.y * v.x, v.y, v.z);
-                    d[2] = unit_div(hi.x * v.x, v.y, v.z);
-                    d[3] = unit_div(hi.y * v.x, v.y, v.z);
+                for (int q = 0; q < 4; ++q) {
+                    const float2 lo = fp8_pair<false>(words[q]), hi = fp8_pair<true>(words[q]);
+                    float* d = u + 16 * j + 4 * q;
+                    d[0] = unit(lo.x);
+                    d[1] = unit(lo.y);
+                    d[2] = unit(hi.x);
+                    d[3] = unit(hi.y);
                 }
             }
+        };
+        if (all_short) {
+            const Recip r = sm.r[id];
+            each_word([&](float c) __attribute__((always_inline)) { return unit_short(c, r); });
+        } else {
+            const float4 v = sm.v[id];
+            each_word([&](float c) __attribute__((always_inline)) { return unit_div(c * v.x, v.y, v.z); });
         }
     };
     // dot with token t's unit vector: lane i of a row expands its dims i, 16 + i, ...
     auto dot = [&](int32_t t) __attribute__((always_inline)) {
-        const float4 v = sm.v[t];
         const uint8_t* row = reinterpret_cast<const uint8_t*>(sm.c[t]) + (lane & 15);
         float a[8];
+        if (all_short) {
+            const Recip r = sm.r[t];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) a[j] = unit_div(fp8_at<0>(row[16 * (j ^ (t & 7))]) * v.x, v.y, v.z);
+            for (int j = 0; j < 8; ++j) a[j] = unit_short(fp8_at<0>(row[16 * (j ^ (t & 7))]), r);
+        } else {
+            const float4 v = sm.v[t];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) a[j] = unit_div(fp8_at<0>(row[16 * (j ^ (t & 7))]) * v.x, v.y, v.z);
+        }
         Acc4 acc;
         dot_units(acc, a, u);
         return acc.total();
@@ -645,12 +653,13 @@ __global__ __launch_bounds__(kQuarter, 3) void build_quarter_kernel(const uint8_
 #pragma unroll
     for (int off = 1; off < 8; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
     const float scale = center_scale(amax);
+    const float inv = 1.0f / scale;  // (a power of two from 2^-22 to 2^120: the products are the quotients)
     uint32_t packed[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-        packed[q] = e4m3_code(mean[4 * q] / scale) | (e4m3_code(mean[4 * q + 1] / scale) << 8) |
-                    (e4m3_code(mean[4 * q + 2] / scale) << 16) |
-                    (e4m3_code(mean[4 * q + 3] / scale) << 24);
+        packed[q] = e4m3_code(mean[4 * q] * inv) | (e4m3_code(mean[4 * q + 1] * inv) << 8) |
+                    (e4m3_code(mean[4 * q + 2] * inv) << 16) |
+                    (e4m3_code(mean[4 * q + 3] * inv) << 24);
     const int32_t center = at / 8;
     uint8_t* cp = centers_out + (b * 2 + center / 64) * V1_PAGE_BYTES;
     *reinterpret_cast<uint4*>(cp + (center % 64) * 128 + 16 * r) = make_uint4(packed[0], packed[1], packed[2], packed[3]);

@@ -190,3 +190,27 @@ def test_build_buckets_out_of_pool_pages_and_empty_batch(mods):
     assert np.array_equal(H(mapping[0]), e_map) and np.array_equal(H(centers[0]), e_centers)
     out = IB.build_buckets(T(pool), T(np.zeros((0, 16), np.int32)), T(np.zeros(0, np.int32)))
     assert all(o.shape[0] == 0 for o in out)
+
+
+def _rescaled(pool, factors):
+    """The pool with its tokens' scales multiplied by `factors` (in token order)."""
+    out = pool.copy()
+    scales = out[:, 8192:].copy().view(np.float32)
+    scales *= np.resize(np.asarray(factors, np.float32), scales.shape)
+    out[:, 8192:] = scales.view(np.uint8)
+    return out
+
+
+# scales that are powers of two take the short unit quotient, wave by wave or quarter by quarter; any other scale, and
+# powers of two outside 2^-40 .. 2^40, the general one
+@pytest.mark.parametrize("factors", [[1.1], [1.0] * 200 + [0.7], [2.0**30, 2.0**-30], [2.0**-60], [1.0] * 64 + [3.0] * 64])
+def test_build_buckets_scales(mods, factors):
+    _, _, IB = mods
+    pool = _rescaled(_pool(31), factors)
+    tables = np.stack([np.random.default_rng(i).permutation(24)[:16] for i in range(3)]).astype(np.int32)
+    starts = np.int32([0, 1024, 4096])
+    perm, tmp, mapping, centers = IB.build_buckets(T(pool), T(tables), T(starts))
+    for b in range(3):
+        e_perm, e_tmp, e_map, e_centers = O.index_build(pool, tables[b], int(starts[b]))
+        assert np.array_equal(H(perm[b]), e_perm) and np.array_equal(H(tmp[b]), e_tmp)
+        assert np.array_equal(H(mapping[b]), e_map) and np.array_equal(H(centers[b]), e_centers)

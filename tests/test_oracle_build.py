@@ -227,3 +227,16 @@ def test_assemble_copies_and_centers():
     np.testing.assert_allclose(dec, mean, rtol=2.0 ** -4, atol=2.0 ** -9 * cs.max())
     amax = np.abs(mean).max(axis=1)
     assert (amax / cs > 224).all() | (amax < 1e-4 * 448).any()  # the scale is the smallest power of two
+
+
+def test_short_unit_quotient_is_the_division():
+    # build.hip's unit_short: fl(c h + fl(c l)) with h = fl(1 / d), l = fl((1 - h d) / d) equals fl(c / d) for every
+    # 4-bit significand c and 24-bit significand d (exponents only scale all terms).  In float64 the residual, the
+    # products and the sum below are exact (at most 52 bits), so each step rounds once, as the FMA does.
+    for first in range(1 << 23, 1 << 24, 1 << 21):
+        d = np.arange(first, first + (1 << 21), dtype=np.float64).astype(np.float32) * np.float32(2.0**-23)
+        h = np.float32(1.0) / d
+        low = (1.0 - h.astype(np.float64) * d).astype(np.float32) / d
+        for c in range(8, 16):
+            short = (c * h.astype(np.float64) + (np.float32(c) * low)).astype(np.float32)
+            assert np.array_equal(short, np.float32(c) / d)
