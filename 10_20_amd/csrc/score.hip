@@ -1360,9 +1360,10 @@ __global__ __launch_bounds__(kPlanThreads) void score_union_plan(ScoreParams p, 
 //   score_pages        the work items, plus one extra grid row that scores the
 //                      overflow pairs one wave per pair.
 constexpr int kPmPages = 8;
-constexpr int kPmWaves = 4;                // waves per work-group
-constexpr bool kPmPrefetch = true;         // the next row's loads issued before the current row
-constexpr int kPmRows = 16 * kPmWaves;     // rows per work item
+constexpr int kPmWaves = 8;                // waves per work-group
+constexpr int kPmRows = 64;                // rows per work item: a wave's (row, page) slots are one per lane
+constexpr int kPmSplit = 2;                // a split item is kPmRows / kPmSplit rows
+static_assert(kPmRows / kPmWaves * kPmPages == kWave && kPmRows % (kPmWaves * kPmSplit) == 0, "slots one per lane");
 constexpr uint32_t kPmNone = 0xffffffffu;
 constexpr int64_t kPmMaxTableBytes = 64ll << 20;
 
@@ -1386,6 +1387,7 @@ struct PmTables {
     int32_t chunks;
     int32_t words;
     int32_t compact;      // chunks of listed pages (else of consecutive pool pages)
+    int32_t whole, split; // chunks whose items are kPmRows rows, and chunks whose items are a kPmSplit-th of that
 };
 
 struct PmLayout {
@@ -1492,18 +1494,62 @@ __global__ __launch_bounds__(256) void score_pages_place(ScoreParams p, PmTables
     for (int i = 0; i < 64; ++i) store_logit(p, row, j * 64 + i, ctx, 0.f);
 }
 
+// One (row, listed page) pair is 4 * HB MFMAs over fragments read from LDS,
+// and per MFMA eight vector operations of direct ReLU: the kernel is bound by
+// vector issue, and what it needs is waves that fill each other's LDS, query
+// and store latencies.  So a work-group is 8 waves over one staged chunk (two
+// work-groups, 16 waves per CU, at most 128 registers): a wave keeps one
+// row's query fragments and weights and half a page's key fragments, each
+// key block's read two blocks ahead, on into the row's next page.  The wave
+// holds the table slots of all its rows in one register (lane i * 8 + k: row
+// i, page k) and walks the listed pairs by the set bits of one ballot.
+// Against 4 waves of a prefetched row and a whole page each (227 registers,
+// two waves per SIMD): 1024 rows x 64 heads listing 542 of 1076 pages 813 K ->
+// 580 K cycles (the whole query 558 -> 491 us), MFMA pipe busy 34 -> 48%; 4096
+// rows x 32 heads listing 108 of 170 pages 169 -> 136 us.  Cutting an item's
+// pairs into equal runs per wave instead of whole rows gained nothing (493 /
+// 142 us), nor did folding five MFMAs after issue (492 / 147 us).
 template <int HB, bool RELU>
-__global__ __launch_bounds__(kWave * kPmWaves) void score_pages(ScoreParams p, PmTables m) {
+__global__ __launch_bounds__(kWave * kPmWaves, 4) void score_pages(ScoreParams p, PmTables m) {
     __shared__ __attribute__((aligned(16))) uint8_t pages[kPmPages][V1_PAGE_BYTES];
     __shared__ uint32_t used_sh;
-    constexpr int kBlock = kWave * kPmWaves;
     const int t = threadIdx.x, l = __lane_id(), wv = __builtin_amdgcn_readfirstlane(t / kWave);
     // B fragment of key block kb of a staged page: key kb*16 + l%16, chunks
     // 2*(l/16) and +1 (stored swizzled, as score_shared stages them)
     const int swz = key_swizzle(l & 15);
     const int boff0 = (l & 15) * 128 + (((2 * (l >> 4)) ^ swz) << 4);
     const int boff1 = (l & 15) * 128 + (((2 * (l >> 4) + 1) ^ swz) << 4);
-    if ((int32_t)blockIdx.y == m.chunks) {
+    // a row's query fragments and weights, through descriptors that end at its
+    // last head: heads past it load as zeros
+    const int qoff = (l & 15) * 128 + 32 * (l >> 4);
+    auto load_row = [&](int64_t row, v8i (&a)[HB], float (&w)[HB][4]) __attribute__((always_inline)) {
+        const auto qr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.q + row * p.heads * 128), 0,
+                                                          p.heads * 128, kRawDword);
+        const auto wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.w + row * p.heads), 0, p.heads * 4,
+                                                          kRawDword);
+#pragma unroll
+        for (int hb = 0; hb < HB; ++hb) {
+            const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(qr, qoff, hb * 2048, 0);
+            const u32x4 z = __builtin_amdgcn_raw_buffer_load_b128(qr, qoff + 16, hb * 2048, 0);
+            a[hb] = v8i{(int)x.x, (int)x.y, (int)x.z, (int)x.w, (int)z.x, (int)z.y, (int)z.z, (int)z.w};
+        }
+        if ((p.heads & 3) == 0) {
+#pragma unroll
+            for (int hb = 0; hb < HB; ++hb) {
+                const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * (l >> 4), hb * 64, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[hb][i] = __uint_as_float(x[i]);
+            }
+        } else {
+#pragma unroll
+            for (int hb = 0; hb < HB; ++hb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    w[hb][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(wr, 16 * (l >> 4) + 4 * i, hb * 64, 0));
+        }
+    };
+    const int32_t y = blockIdx.y;
+    if (y == m.whole + m.split * kPmSplit) {
         // overflow pairs: one wave per pair, the page read straight from memory
         const uint32_t n = *m.count;
         for (uint32_t e = blockIdx.x * kPmWaves + wv; e < n; e += gridDim.x * kPmWaves) {
@@ -1513,8 +1559,7 @@ __global__ __launch_bounds__(kWave * kPmWaves) void score_pages(ScoreParams p, P
             const int32_t page = page_of(p, row, slot);
             v8i a[HB], b[4];
             float w[HB][4];
-            load_q<HB>(p, row, a);
-            load_w<HB>(p, row, w);
+            load_row(row, a, w);
             const uint8_t* base = p.kv + (int64_t)max(page, 0) * V1_PAGE_BYTES;
 #pragma unroll
             for (int kb = 0; kb < 4; ++kb) {
@@ -1529,20 +1574,27 @@ __global__ __launch_bounds__(kWave * kPmWaves) void score_pages(ScoreParams p, P
         }
         return;
     }
-    const int32_t c = blockIdx.y;
-    const int64_t r0 = (int64_t)blockIdx.x * kPmRows;
-    const uint32_t* tab = m.table + (int64_t)c * p.rows * kPmPages;
-    // pages of the chunk that the block's rows list
+    // Chunks are taken from the last one down, and the last m.split of them
+    // taken are cut into items of half the rows (see v1_score).
+    const bool whole_item = y < m.whole;
+    const int32_t ys = y - m.whole;
+    const int32_t c = m.whole + m.split - 1 - (whole_item ? y : m.whole + ys / kPmSplit);
+    const int32_t wave_rows = whole_item ? kPmRows / kPmWaves : kPmRows / kPmWaves / kPmSplit;
+    const int64_t r0 = (int64_t)blockIdx.x * kPmRows + (whole_item ? 0 : ys % kPmSplit * (kPmRows / kPmSplit)) +
+                       wv * wave_rows;
+    const int32_t nrows = (int32_t)max<int64_t>(0, min<int64_t>(wave_rows, (int64_t)p.rows - r0));
     if (t == 0) used_sh = 0;
+    uint32_t slots = kPmNone;
+    if (l < nrows * kPmPages) slots = m.table[((int64_t)c * p.rows + r0) * kPmPages + l];
+    uint64_t pairs = __builtin_amdgcn_ballot_w64(slots != kPmNone);
+    // pages of the chunk that the item's rows list
+    uint64_t fold = pairs | (pairs >> 32);
+    fold |= fold >> 16;
+    const uint32_t mine = (uint32_t)(fold | (fold >> 8)) & 0xffu;
     __syncthreads();
-    uint32_t used = 0;
-    for (int e = t; e < kPmRows * kPmPages; e += kBlock) {
-        const int64_t r = r0 + e / kPmPages;
-        if (r < p.rows && tab[r * kPmPages + e % kPmPages] != kPmNone) used |= 1u << (e % kPmPages);
-    }
-    if (used) atomicOr(&used_sh, used);
+    if (l == 0 && mine) atomicOr(&used_sh, mine);
     __syncthreads();
-    used = __builtin_amdgcn_readfirstlane(used_sh);
+    const uint32_t used = __builtin_amdgcn_readfirstlane(used_sh);
     if (used == 0) return;
     // stage the listed pages: per page eight 1 KiB key chunks and 256 bytes
     // of scales, the 72 loads dealt to the waves in turn
@@ -1563,114 +1615,66 @@ __global__ __launch_bounds__(kWave * kPmWaves) void score_pages(ScoreParams p, P
         }
     }
     V1_PAGE_BARRIER(0);
-    // Rows of this wave: r0 + wv, r0 + wv + 4, ...  The next row's table
-    // slots, query fragments, weights and length are loaded before the
-    // current row is computed (two register sets, used in turn); every load
-    // is issued from a clamped index and every row issues exactly kPmPages
-    // logit stores (range-checked buffer stores: a page the row does not list
-    // gets a descriptor of length 0), so the wait for a row's data is an
-    // exact count and never drains the next row's loads.
-    const auto tab_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(tab), 0,
-                                                          (int32_t)(p.rows * kPmPages * 4), kRawDword);
-    const auto ctx_rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(p.ctx), 0, p.rows * 4, kRawDword);
-    const auto none_rs = __builtin_amdgcn_make_buffer_rsrc(p.logits, 0, 0, kRawDword);
-    struct RowData {
-        u32x4 s[kPmPages / 4];
+    constexpr int kN = 4 * HB, kLag = 3;
+    while (pairs) {
+        const int i = __builtin_ctzll(pairs) / kPmPages;
+        const int64_t row = r0 + i;
+        uint32_t todo = (uint32_t)(pairs >> (i * kPmPages)) & 0xffu;  // the row's listed pages
+        pairs &= ~(0xffull << (i * kPmPages));
         v8i a[HB];
         float w[HB][4];
-        int32_t ctx;
-    };
-    // Whole head blocks (heads a multiple of 16): the query fragments and
-    // weights load without the per-lane range selects (a row past the end
-    // reads the last row, whose logits it never stores).
-    const bool whole = (p.heads & 15) == 0;
-    auto fetch = [&](int64_t row, RowData& d) __attribute__((always_inline)) {
-        const int32_t rc = (int32_t)min(row, (int64_t)p.rows - 1);
+        load_row(row, a, w);
+        const int32_t ctx = min(p.ctx[row], p.max_context_len);
+        const int32_t end = p.clean ? p.max_context_len : ctx;
+        float* const out = p.logits + row * p.logits_stride;
+        int k = __builtin_ctz(todo);
+        const uint8_t* at = pages[0] + k * V1_PAGE_BYTES;
+        v8i b[2];
+        auto frag = [&](const uint8_t* page, int kb, v8i& f) __attribute__((always_inline)) {
+            const u32x4 x = *reinterpret_cast<const u32x4*>(page + kb * 2048 + boff0);
+            const u32x4 z = *reinterpret_cast<const u32x4*>(page + kb * 2048 + boff1);
+            f = v8i{(int)x.x, (int)x.y, (int)x.z, (int)x.w, (int)z.x, (int)z.y, (int)z.z, (int)z.w};
+        };
+        frag(at, 0, b[0]);
+        frag(at, 1, b[1]);
+        for (;;) {
+            todo &= todo - 1u;
+            const int kn = todo ? __builtin_ctz(todo) : k;  // (past the row's last page: read once more, not used)
+            const uint8_t* next = pages[0] + kn * V1_PAGE_BYTES;
+            const float scale = reinterpret_cast<const float*>(at + 8192)[l];
+            float s[4];
+            v4f d[kLag + 1];
+            // (page_partials_lag's products in its order: the same values bit for bit)
 #pragma unroll
-        for (int i = 0; i < kPmPages / 4; ++i)
-            d.s[i] = __builtin_amdgcn_raw_buffer_load_b128(tab_rs, rc * kPmPages * 4 + 16 * i, 0, 0);
-        if (whole) {
-#pragma unroll
-            for (int hb = 0; hb < HB; ++hb) {
-                const int h = hb * 16 + (l & 15);
-                const u32x4* src = reinterpret_cast<const u32x4*>(p.q + ((int64_t)rc * p.heads + h) * 128 + 32 * (l >> 4));
-                const u32x4 x = src[0], y = src[1];
-                d.a[hb] = v8i{(int)x.x, (int)x.y, (int)x.z, (int)x.w, (int)y.x, (int)y.y, (int)y.z, (int)y.w};
-                const v4f wv4 = *reinterpret_cast<const v4f*>(p.w + (int64_t)rc * p.heads + hb * 16 + 4 * (l >> 4));
-#pragma unroll
-                for (int i = 0; i < 4; ++i) d.w[hb][i] = wv4[i];
-            }
-        } else {
-            load_q<HB>(p, row, d.a);
-            load_w<HB>(p, row, d.w);
-        }
-        d.ctx = (int32_t)__builtin_amdgcn_raw_buffer_load_b32(ctx_rs, rc * 4, 0, 0);
-    };
-    auto run = [&](int64_t row, const RowData& d) __attribute__((always_inline)) {
-        uint32_t slot[kPmPages];
-#pragma unroll
-        for (int k = 0; k < kPmPages; ++k) slot[k] = d.s[k / 4][k % 4];
-        const int32_t ctx = min(__builtin_amdgcn_readfirstlane(d.ctx), p.max_context_len);
-        const bool live_row = row < p.rows;
-#pragma unroll
-        for (int k = 0; k < kPmPages; ++k) {
-            const uint32_t sk = __builtin_amdgcn_readfirstlane(slot[k]);
-            const bool live = live_row && sk != kPmNone;
-            if (!live) {
-                // (the store count stays fixed: a zero-length descriptor drops it)
-                __builtin_amdgcn_raw_buffer_store_b32(0u, none_rs, 0, 0, 0);
-                continue;
-            }
-            float v = 0.f;
-            {
-                v8i b[4];
-#pragma unroll
-                for (int kb = 0; kb < 4; ++kb) {
-                    const u32x4 x = *reinterpret_cast<const u32x4*>(pages[k] + kb * 2048 + boff0);
-                    const u32x4 y = *reinterpret_cast<const u32x4*>(pages[k] + kb * 2048 + boff1);
-                    b[kb] = v8i{(int)x.x, (int)x.y, (int)x.z, (int)x.w, (int)y.x, (int)y.y, (int)y.z, (int)y.w};
+            for (int idx = 0; idx < kN + kLag; ++idx) {
+                if (idx < kN) {
+                    const int kb = idx / HB;
+                    d[idx % (kLag + 1)] = mfma_fp8(a[idx % HB], b[kb & 1]);
+                    if (idx % HB == HB - 1) frag(kb < 2 ? at : next, (kb + 2) & 3, b[kb & 1]);
                 }
-                float part[4];
-                page_partials_lag<HB, RELU>(d.a, b, d.w, part);
-                v = reduce_scatter4(part) * reinterpret_cast<const float*>(pages[k] + 8192)[l];
+                const int j = idx - kLag;
+                if (j >= 0) {
+                    const v4f x = d[j % (kLag + 1)];
+                    const int kb = j / HB, hb = j % HB;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float prev = (hb == 0 && e == 0) ? 0.f : s[kb];
+                        s[kb] = fmaf(w[hb][e], RELU ? relu(x[e]) : x[e], prev);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
+            const float v = reduce_scatter4(s) * scale;
             // columns [col, col + 64) of the row: logits below its context,
             // -inf from there to max_context_len with clean_logits
-            const int32_t col = (int32_t)sk * 64;
-            const int32_t end = (p.clean ? p.max_context_len : ctx) - col;
-            const int32_t lim = __builtin_amdgcn_readfirstlane(end > 0 ? (end < 64 ? end : 64) : 0);
-            // (the row's address made scalar explicitly: the descriptor must be)
-            const uint64_t at = reinterpret_cast<uint64_t>(p.logits + min(row, (int64_t)p.rows - 1) * p.logits_stride + col);
-            const uint64_t at_s = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) |
-                                  (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at);
-            const auto rs = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<float*>(at_s), 0, lim * 4, kRawDword);
+            const int32_t col = __builtin_amdgcn_readlane((int)slots, i * kPmPages + k) * 64;
+            const int32_t lim = __builtin_amdgcn_readfirstlane(max(0, min(64, end - col)));
+            const auto rs = __builtin_amdgcn_make_buffer_rsrc(out + col, 0, lim * 4, kRawDword);
             __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(l < ctx - col ? v : -__builtin_huge_valf()), rs, l * 4,
                                                   0, 0);
-        }
-    };
-    constexpr int kSteps = kPmRows / kPmWaves;
-    static_assert(kSteps % 2 == 0, "rows taken in pairs");
-    if constexpr (kPmPrefetch) {
-        RowData d0, d1;
-        fetch(r0 + wv, d0);
-#pragma unroll 1
-        for (int i = 0; i < kSteps; i += 2) {
-            const int64_t ra = r0 + wv + kPmWaves * i;
-            if (ra >= p.rows) break;
-            fetch(ra + kPmWaves, d1);
-            run(ra, d0);
-            if (ra + kPmWaves >= p.rows) break;
-            fetch(ra + 2 * kPmWaves, d0);
-            run(ra + kPmWaves, d1);
-        }
-    } else {
-#pragma unroll 1
-        for (int i = 0; i < kSteps; ++i) {
-            const int64_t ra = r0 + wv + kPmWaves * i;
-            if (ra >= p.rows) break;
-            RowData d0;
-            fetch(ra, d0);
-            run(ra, d0);
+            if (!todo) break;
+            k = kn;
+            at = next;
         }
     }
 }
@@ -2017,12 +2021,20 @@ extern "C" int v1_score(const v1_score_args* a, void* stream) {
         (reinterpret_cast<uintptr_t>(a->workspace) & 255) == 0) {
         const PmLayout L = pm_layout(a->rows, a->max_context_len, a->kv_blocks);
         uint8_t* ws = static_cast<uint8_t*>(a->workspace);
+        // Chunks are dispatched from the pool's end down: a fine pool ends in
+        // its sink and tail pages, which every row lists, so the heaviest
+        // items start first; and the last round of items (about two
+        // work-groups per CU) is cut in half, so that the CUs end closer
+        // together.  Halves against none and quarters: 491 / 495 / 491 us for
+        // a 1024-row query, 136 / 139 / 142 us for 4096 rows of 170 pages.
+        const int64_t blocks = cdiv(a->rows, kPmRows);
+        const int32_t split = (int32_t)std::min<int64_t>(L.chunks, cdiv(2 * (int64_t)v1::device_cus(), blocks));
         const PmTables m{reinterpret_cast<uint32_t*>(ws + L.table), reinterpret_cast<uint32_t*>(ws + L.overflow),
                          reinterpret_cast<uint32_t*>(ws + L.count), reinterpret_cast<uint32_t*>(ws + L.bits),
                          reinterpret_cast<uint32_t*>(ws + L.word_base), reinterpret_cast<int32_t*>(ws + L.listed),
                          L.table_words, L.chunks, L.words,
                          // a pool more than twice a row's pages (listed pages spread thin)
-                         a->kv_blocks > 2 * cdiv(a->max_context_len, 64)};
+                         a->kv_blocks > 2 * cdiv(a->max_context_len, 64), L.chunks - split, split};
         const int64_t clear_wgs = std::max<int64_t>(1, std::min<int64_t>(cdiv(L.table_words, 256), 4 * (int64_t)v1::device_cus()));
         hipLaunchKernelGGL(score_pages_clear, dim3((uint32_t)clear_wgs), dim3(256), 0, st, m);
         int rc = V1_LAUNCHED("score_pages_clear");
@@ -2039,7 +2051,7 @@ extern "C" int v1_score(const v1_score_args* a, void* stream) {
                            dim3(256), 0, st, p, m);
         rc = V1_LAUNCHED("score_pages_place");
         if (rc != V1_OK) return rc;
-        launch_hb<Pages>(hb, a->relu != 0, dim3((uint32_t)cdiv(a->rows, kPmRows), (uint32_t)L.chunks + 1), st, p, m);
+        launch_hb<Pages>(hb, a->relu != 0, dim3((uint32_t)blocks, (uint32_t)(m.whole + m.split * kPmSplit + 1)), st, p, m);
         return V1_LAUNCHED("score_pages");
     }
     // Per-row tables of more than 512 rows with a large enough workspace:

@@ -284,3 +284,30 @@ def test_page_major_bitwise_equals_row_kernel(dev, heads, relu, pool_pages):
     pool, tab = _padded(native, table, width)
     if relu:
         assert_scores_rel(both.astype(np.float64), O.paged_logits(q8, w, pool, tab, lens, width))
+
+
+@pytest.mark.parametrize("rows,heads,relu", [(4161, 33, True), (4161, 64, True), (577, 62, True), (2049, 48, False),
+                                             (1000, 17, True)])
+def test_page_major_items_bitwise_equal_union_plan(dev, rows, heads, relu):
+    """Page-major items of 64 rows and of the half of that at the end of the
+    grid, a last item of a few rows or one, and heads that end inside a
+    16-byte load of the weights (33, 62, 17): the bits of the page-union plan,
+    which takes the same products in the same order.  170 pages are 22 chunks:
+    with 4161 rows 8 of them are halved, with 577 or 1000 all of them."""
+    g = np.random.default_rng(rows + heads)
+    q8, w = _queries(g, rows, heads, heads)
+    if not relu:
+        w *= np.where(g.random(w.shape) < 0.5, -1, 1).astype(np.float32)
+    k8, ks = W.quantize_rows(g.standard_normal((170 * 64, 128), dtype=np.float32))
+    native = W.pack_pages(k8, ks)
+    table = g.random((rows, 170)).argsort(1)[:, :90].astype(np.int32)
+    lens = g.integers(0, 90 * 64 + 1, rows).astype(np.int32)
+    out = []
+    prev = SC.page_major(True)
+    try:
+        for on in (True, False):
+            SC.page_major(on)
+            out.append(_run(dev, q8, w, native, table, lens, 90 * 64, relu, True).astype(np.float32))
+    finally:
+        SC.page_major(prev)
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
