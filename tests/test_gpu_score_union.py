@@ -311,3 +311,36 @@ def test_page_major_items_bitwise_equal_union_plan(dev, rows, heads, relu):
     finally:
         SC.page_major(prev)
     assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,pool_pages,blocks", [(520, 20000, 40), (513, 90, 90), (600, 33, 64)])
+def test_page_major_pair_table_sizes_and_repeats(dev, rows, pool_pages, blocks):
+    """The pair table gathered in LDS for a pool past 64 KiB of it, an ordinary
+    one and one of a few chunks; rows that list one page in every slot (more
+    repeats than the overflow rows' waves take in a step), negative entries
+    and entries past the pool, and rows of no length: the bits of the
+    page-union plan."""
+    g = np.random.default_rng(rows + blocks)
+    q8, w = _queries(g, rows, 20, 20)
+    k8, ks = W.quantize_rows(g.standard_normal((pool_pages * 64, 128), dtype=np.float32))
+    native = W.pack_pages(k8, ks)
+    shared = g.permutation(pool_pages)[:min(pool_pages, 60)]
+    table = shared[g.random((rows, 64)).argsort(1)[:, :blocks] % len(shared)] if blocks <= 64 else \
+        g.random((rows, pool_pages)).argsort(1)[:, :blocks]
+    table = np.ascontiguousarray(table, np.int32)
+    table[5] = table[5, 0]
+    table[rows - 1] = table[rows - 1, 0]
+    table[7, ::3] = -1
+    table[8, 1::4] = pool_pages
+    lens = g.integers(1, blocks * 64 + 1, rows).astype(np.int32)
+    lens[[5, rows - 1]] = blocks * 64
+    lens[9:12] = 0
+    out = []
+    prev = SC.page_major(True)
+    try:
+        for on in (True, False):
+            SC.page_major(on)
+            out.append(_run(dev, q8, w, native, table, lens, blocks * 64 + 100, True, True).astype(np.float32))
+    finally:
+        SC.page_major(prev)
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
