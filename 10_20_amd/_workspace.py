@@ -20,9 +20,8 @@ _retired = []
 
 def _key(device, tag, stream):
     index = device.index if device.index is not None else torch.cuda.current_device()
-    if stream is None:
-        stream = torch.cuda.current_stream(index)
-    return index, stream.cuda_stream, tag
+    raw = torch._C._cuda_getCurrentRawStream(index) if stream is None else stream.cuda_stream
+    return index, raw, tag
 
 
 def workspace(device, nbytes, tag="default", stream=None):

@@ -76,7 +76,7 @@ def gather_rows(pool, ids, out, table=None, page_bits=0):
         raise ValueError("gather_rows: pool must be a uint8 [rows, row_bytes] tensor with unit inner stride")
     rows, top = ids.shape
     row_bytes = pool.shape[1]
-    if tuple(out.shape) != (rows, top, row_bytes) or out.dtype != torch.uint8 or not out.is_contiguous():
+    if out.shape != (rows, top, row_bytes) or out.dtype != torch.uint8 or not out.is_contiguous():
         raise ValueError("gather_rows: out must be a contiguous uint8 [rows, top, row_bytes] tensor")
     if ids.dtype != torch.int32 or ids.stride(1) != 1:
         raise ValueError("gather_rows: ids must be int32 with unit inner stride")

@@ -22,14 +22,19 @@ def _need(cond, msg):
 
 
 def _i32(t, shape, name):
+    # (the messages are made on failure alone: formatting them costs more than the checks)
+    if t.dtype == torch.int32 and t.shape == shape and (t.is_contiguous() or t.numel() == 0):
+        return
     _need(t.dtype == torch.int32, f"{name} must be int32")
-    _need(tuple(t.shape) == tuple(shape), f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
-    _need(t.is_contiguous() or t.numel() == 0, f"{name} must be contiguous")
+    _need(t.shape == shape, f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
+    _need(False, f"{name} must be contiguous")
 
 
 def _selected(t, B, name="selected"):
-    _need(t.dtype in (torch.int32, torch.int64), f"{name} must be int32 or int64")
-    _need(t.dim() == 2 and t.shape[0] == B and t.is_contiguous(), f"{name} must be a contiguous [batch, take] tensor")
+    if t.dtype not in (torch.int32, torch.int64):
+        _need(False, f"{name} must be int32 or int64")
+    if not (t.dim() == 2 and t.shape[0] == B and t.is_contiguous()):
+        _need(False, f"{name} must be a contiguous [batch, take] tensor")
     return 32 if t.dtype == torch.int32 else 64
 
 

@@ -41,7 +41,7 @@ def fp8_paged_mqa_logits(q, kv_cache, weights, context_lens, block_table, schedu
     if q.dim() != 3 or q.shape[2] != 128 or q.element_size() != 1 or not q.is_contiguous():
         raise ValueError("q must be a contiguous [rows, heads, 128] FP8 tensor")
     rows, heads = q.shape[0], q.shape[1]
-    if weights.dtype != torch.float32 or tuple(weights.shape) != (rows, heads) or not weights.is_contiguous():
+    if weights.dtype != torch.float32 or weights.shape != (rows, heads) or not weights.is_contiguous():
         raise ValueError("weights must be a contiguous float32 [rows, heads] tensor")
     lens = context_lens.reshape(-1)
     if lens.dtype != torch.int32 or lens.numel() != rows or not lens.is_contiguous():
