@@ -67,14 +67,10 @@ struct ScoreParams {
     int32_t relu;
     int32_t clean;
     const uint8_t* pieces;  // per-query records from score_prep (shared-table kernel)
-    int32_t nchunks;        // shared-table kernel: chunks of kChunkPages pages over max_context_len
+    int32_t nchunks;        // shared-table kernel: chunks of chunk_pages pages over max_context_len
+    int32_t chunk_pages;    // shared-table kernel: kChunkPages, or less where that leaves work-groups idle
     int32_t groups;         // shared-table kernel: 8-query row groups
-    int32_t items;          // shared-table kernel: groups x levels
-    uint32_t* work;         // shared-table kernel: next work item (zeroed by score_prep)
-    int32_t bulk;           // shared-table kernel: levels of full-size ranges (chunks [L*F, (L+1)*F))
-    int32_t full;           // shared-table kernel: F, the chunks of a full-size range
-    int32_t lvl_start[16];  // shared-table kernel: chunk range of each later level's items
-    int32_t lvl_chunks[16];
+    uint32_t* work;         // [0] next work item (zeroed by score_prep), [1] shared-table kernel: chunks of a full range
     uint32_t* exact_pages;  // shared-table ReLU path: per row, a bitmap of pages for score_exact
     int32_t exact_words;    // 32-bit words per row of exact_pages (score_exact)
     // union form (per-row tables through the page ring), built by score_union_plan:
@@ -87,7 +83,6 @@ struct ScoreParams {
     int32_t u_level_stride;
     const int32_t* row_filter;  // score_rows: rows whose entry is 0 are skipped (nullptr: every row)
 };
-constexpr int kMaxLevels = 16;
 
 // ---------------------------------------------------------- linear term
 // relu(x) = (x + |x|) / 2, so  sum_h w_h relu(q_h . k)
@@ -144,13 +139,44 @@ __device__ __forceinline__ float wave_all(float v, Op op) {
     return op(op(row(0), row(16)), op(row(32), row(48)));
 }
 
+// Chunks of a full range of score_shared's work items (work[1]), from the
+// longest context of the batch: about one range per work-group, at most
+// kMaxRange of them.  One range is one prologue, 6-7 us of dependent loads;
+// two half as long cost 2000 rows of 64 heads x 8000 keys 130 us against 114,
+// and a 1024-row query with 126 center pages 15 us more.  max_context_len in place of the longest
+// context would leave work-groups idle wherever it is a capacity and not a length.
+struct RangePlan {
+    const int32_t* ctx;  // nullptr: no plan, no work-group for it
+    int32_t max_context_len, chunk_pages, groups, wgs, max_range;
+};
+__device__ void plan_ranges(const RangePlan& plan, int32_t rows, uint32_t* work) {
+    __shared__ int32_t part[256 / kWave];
+    int32_t longest = 0;
+#pragma unroll 4
+    for (int32_t r = threadIdx.x; r < rows; r += 256) longest = max(longest, plan.ctx[r]);
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) longest = max(longest, __shfl_xor(longest, d));
+    if (__lane_id() == 0) part[threadIdx.x / kWave] = longest;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    longest = min(max(max(part[0], part[1]), max(part[2], part[3])), plan.max_context_len);
+    const int64_t keys = 64 * (int64_t)plan.chunk_pages;
+    const int64_t chunks = (longest + keys - 1) / keys;
+    work[1] = (uint32_t)max<int64_t>(1, min<int64_t>(plan.max_range, plan.groups * chunks / plan.wgs));
+}
+
 // One wave per query row: q' = sum_h w_h q_h split into its pieces, and the
 // record described above.  relu: 1 the fold (halved weights, pieces, the
 // exact-path threshold); 0 (no ReLU) or 2 (ReLU taken directly, one head
 // block) the weights alone.
 __global__ __launch_bounds__(256) void score_prep(const uint8_t* q, const float* w, int32_t rows, int32_t heads,
                                                   int32_t relu, uint8_t* out, uint32_t* work, uint32_t* exact_pages,
-                                                  int32_t exact_words, uint32_t* clear, int32_t nclear) {
+                                                  int32_t exact_words, uint32_t* clear, int32_t nclear,
+                                                  RangePlan plan) {
+    if (plan.ctx != nullptr && blockIdx.x == gridDim.x - 1) {
+        plan_ranges(plan, rows, work);
+        return;
+    }
     const int64_t row = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int l = __lane_id();
     if (blockIdx.x == 0 && threadIdx.x == 0) *work = 0u;  // the work counter of score_shared
@@ -381,7 +407,8 @@ __device__ __forceinline__ void dma4(const i32x4& rs, int32_t voff, uint32_t lds
 // and page ids are loaded once per item; each page's logits are stored from
 // registers as soon as they are computed.
 constexpr int kMaxRangePages = 256;
-constexpr int kMarkWords = kMaxRangePages / 32 + 1;  // an item's pages start at a multiple of 16
+constexpr int kMarkWords = kMaxRangePages / 32 + 1;  // an item's pages start at any bit of the first word
+static_assert(31 + kMaxRangePages <= 32 * kMarkWords, "an item's marks");
 
 // Union form (per-row tables): an item is a range of at most kUnionRange of a
 // group's union entries (one per lane of a wave); items are listed per level,
@@ -435,8 +462,20 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
         for (int i = t; i < kQueriesPerGroup * kMarkWords; i += kBlock) marks[i] = 0u;
     // union items per level (final before this kernel starts)
     int32_t lvl_n[UNION ? kUnionLevels : 1];
-    int32_t total_items = p.items;
-    if constexpr (UNION) {
+    // Shared tables: every group's ranges of `full` chunks first (`bulk` of
+    // them), then the rest of its chunks in ranges that halve in size, so that
+    // the last ones taken are short and the work-groups end together.
+    int32_t total_items, full = 0, bulk = 0;
+    auto range_chunks = [&](int32_t begin) __attribute__((always_inline)) {
+        return min((p.nchunks - begin + 1) / 2, full);
+    };
+    if constexpr (!UNION) {
+        full = __builtin_amdgcn_readfirstlane((int32_t)p.work[1]);
+        bulk = p.nchunks > 2 * full ? __builtin_amdgcn_readfirstlane((p.nchunks - full) / full) : 0;
+        int32_t levels = bulk;
+        for (int32_t c = bulk * full; c < p.nchunks; c += range_chunks(c)) ++levels;
+        total_items = p.groups * levels;
+    } else {
         total_items = 0;
 #pragma unroll
         for (int L = 0; L < kUnionLevels; ++L) {
@@ -444,11 +483,16 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
             total_items += lvl_n[L];
         }
     }
+  // A work-group's first item is its own number, and further ones are drawn
+  // from the counter (which score_prep leaves at zero): where items are short,
+  // behind the current item's first page loads, so that neither the next item
+  // nor the work-group's end waits on an atomic alone.  Long ones are drawn
+  // when the current one is done: held from its start, they leave the
+  // work-groups less even (32K keys x 4096 rows 780 -> 801 us).
+  const bool ahead = !UNION && full == 1;
+  if (t == 0) item_sh = (int32_t)blockIdx.x;
   for (;;) {
-    // every wave has finished the previous item (its LDS is free) when the
-    // next one is drawn
-    __syncthreads();
-    if (t == 0) item_sh = (int32_t)atomicAdd(p.work, 1u);
+    // every wave has finished the previous item (its LDS is free)
     __syncthreads();
     const int32_t item = __builtin_amdgcn_readfirstlane(item_sh);
     if (item >= total_items) break;
@@ -470,9 +514,13 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
     } else {
         group = item % p.groups;
         const int32_t level = item / p.groups;
-        const int32_t c_begin = level < p.bulk ? level * p.full : p.lvl_start[level - p.bulk];
-        nchunk = level < p.bulk ? p.full : p.lvl_chunks[level - p.bulk];
-        page_begin = c_begin * kChunkPages;
+        int32_t c_begin = min(level, bulk) * full;
+        nchunk = level < bulk ? full : range_chunks(c_begin);
+        for (int32_t k = bulk; k < level; ++k) {
+            c_begin += nchunk;
+            nchunk = range_chunks(c_begin);
+        }
+        page_begin = c_begin * p.chunk_pages;
     }
     const int64_t row0 = (int64_t)group * kQueriesPerGroup;
     const int32_t grows = (int32_t)min<int64_t>(kQueriesPerGroup, (int64_t)p.rows - row0);  // rows of the group
@@ -551,24 +599,25 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
 #pragma unroll
     for (int q = 0; q < QPW; ++q) ctx[q] = __builtin_amdgcn_readlane(lane_ctx, wv * QPW + q);
     // pages of the range below the group's longest context (union: every entry)
-    const int32_t npages = UNION ? ulen : max(0, min(nchunk * kChunkPages, (max_ctx + 63) / 64 - page_begin));
+    const int32_t npages = UNION ? ulen : max(0, min(nchunk * p.chunk_pages, (max_ctx + 63) / 64 - page_begin));
 
     // Pages of the item past the group's longest context are computed by
     // nobody: with clean_logits their columns below max_context_len get -inf.
     // (Union: the plan fills the columns past each row's last page.)
     auto fill_rest = [&](int32_t from_page) __attribute__((always_inline)) {
         if (UNION || !p.clean) return;
-        for (int32_t pg = from_page; pg < nchunk * kChunkPages; ++pg) {
+        for (int32_t pg = from_page; pg < nchunk * p.chunk_pages; ++pg) {
 #pragma unroll
             for (int q = 0; q < QPW; ++q)
                 store_logit(p, row0 + wv * QPW + q, (page_begin + pg) * 64 + l, ctx[q], 0.f);
         }
     };
+    __syncthreads();  // page ids in LDS; every wave has read item_sh
     if (npages == 0) {
+        if (t == 0) item_sh = (int32_t)(gridDim.x + atomicAdd(p.work, 1u));
         fill_rest(0);
         continue;
     }
-    __syncthreads();  // page ids in LDS
 
     // per-lane load offsets (into the page) of this wave's loads
     int32_t voff[kKeyDma];
@@ -600,6 +649,8 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
         for (int j = 0; j < 2 * kWin; ++j)
             issue(ring[j], j < npages ? __builtin_amdgcn_readfirstlane(pids[j]) : -1);
     }
+    uint32_t drawn = 0u;
+    if (ahead && t == 0) drawn = atomicAdd(p.work, 1u);
 
     // B fragment of key block kb: key kb*16 + l%16, chunks 2*(l/16) and +1;
     // plus the scale of key l
@@ -846,6 +897,7 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
     // loaded above are complete before the loop, so no wait for them is
     // placed inside it.  (It also covers the first pages.)
     __builtin_amdgcn_s_waitcnt(0);
+    if (ahead && t == 0) item_sh = (int32_t)(gridDim.x + drawn);
     V1_PAGE_BARRIER(0);
 #pragma unroll
     for (int q = 0; q < QPW; ++q)
@@ -903,6 +955,7 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
         }
     }
     V1_PAGE_BARRIER(0);  // the page buffers are reused by the next item
+    if (!ahead && t == 0) item_sh = (int32_t)(gridDim.x + atomicAdd(p.work, 1u));
     fill_rest(npages);
     if constexpr (UNION) {
         // marked pages to the rows' page bitmaps, at each row's table slot
@@ -1976,35 +2029,24 @@ extern "C" int v1_score(const v1_score_args* a, void* stream) {
         V1_REQUIRE(a->workspace != nullptr && a->workspace_bytes >= need, "score: workspace of %lld bytes required",
                    (long long)need);
         V1_REQUIRE((reinterpret_cast<uintptr_t>(a->workspace) & 15) == 0, "score: workspace must be 16-byte aligned");
-        // Work items: each row group's chunks cut into ranges that halve in
-        // size (at most kMaxRangePages pages), all groups' largest ranges
-        // first; work-groups pull them in that order, so the last ones taken
-        // are short and the work-groups end together.  With few row groups
-        // the full range shrinks so that the chunks make at least two items
-        // per work-group: 1024 queries over 128 center pages (16 chunks of
-        // max_context_len, 8 of them real) otherwise put each group's work in
-        // one 128-page item on 128 of the 512 work-groups.
+        // Work items: each row group's chunks cut into ranges (plan_ranges,
+        // and score_shared's own comment) that work-groups take largest first.
         const int64_t groups = cdiv(a->rows, kQueriesPerGroup);
         const int64_t wgs = 2 * (int64_t)v1::device_cus();
-        const int64_t full = std::max<int64_t>(
-            1, std::min<int64_t>(kMaxRangePages / kChunkPages, groups * (int64_t)chunks / (2 * wgs)));
-        p.full = (int32_t)full;
-        p.bulk = (int32_t)((int64_t)chunks > 2 * full ? ((int64_t)chunks - full) / full : 0);
-        int nlevels = 0;
-        for (int64_t c = (int64_t)p.bulk * full; c < (int64_t)chunks;) {
-            const int64_t left = (int64_t)chunks - c;
-            const int64_t size = std::min<int64_t>(left == 1 ? 1 : (left + 1) / 2, full);
-            p.lvl_start[nlevels] = (int32_t)c;
-            p.lvl_chunks[nlevels] = (int32_t)size;
-            ++nlevels;
-            c += size;
+        const int64_t pages = cdiv(a->max_context_len, 64);
+        int64_t chunks = cdiv(pages, kChunkPages);
+        p.chunk_pages = kChunkPages;
+        if (groups * chunks < wgs && groups * pages > wgs) {
+            // fewer chunks than work-groups: shorter ones (4 pages fill the
+            // page ring), an equal count of them per row group: 100 rows of
+            // 64 heads x 20000 keys 44 -> 41 us, 600 of 32 x 5003 38 -> 37
+            p.chunk_pages = (int32_t)std::max<int64_t>(kStages, cdiv(pages, wgs / groups));
+            chunks = cdiv(pages, p.chunk_pages);
         }
-        static_assert(kMaxLevels >= 8, "the halving tail of at most 2 full ranges has at most 7 levels");
         p.nchunks = (int32_t)chunks;
         p.groups = (int32_t)groups;
-        const int64_t items = groups * ((int64_t)p.bulk + nlevels);
+        const int64_t items = groups * chunks;  // (ranges of one chunk: the most there can be)
         V1_REQUIRE(items < (1ll << 31) - (1ll << 20), "score: too many work items");
-        p.items = (int32_t)items;
         uint8_t* ws = static_cast<uint8_t*>(a->workspace);
         p.pieces = ws;
         p.work = reinterpret_cast<uint32_t*>(ws + (int64_t)a->rows * kPieceRowBytes);
@@ -2013,9 +2055,11 @@ extern "C" int v1_score(const v1_score_args* a, void* stream) {
         // ReLU taken directly with one head block (score_shared's kFold)
         const bool fold = a->relu && hb > 1;
         p.exact_words = fold ? exact_words(a->max_context_len) : 0;
-        const dim3 row_waves((uint32_t)cdiv(a->rows, 4));
-        hipLaunchKernelGGL(score_prep, row_waves, dim3(256), 0, st, a->q, a->weights, a->rows, a->heads,
-                           fold ? 1 : a->relu ? 2 : 0, ws, p.work, p.exact_pages, p.exact_words, nullptr, 0);
+        const dim3 row_waves((uint32_t)cdiv(a->rows, 4)), prep_waves(row_waves.x + 1);
+        const RangePlan plan{a->context_lens, a->max_context_len, p.chunk_pages, p.groups, (int32_t)wgs,
+                             kMaxRangePages / kChunkPages};
+        hipLaunchKernelGGL(score_prep, prep_waves, dim3(256), 0, st, a->q, a->weights, a->rows, a->heads,
+                           fold ? 1 : a->relu ? 2 : 0, ws, p.work, p.exact_pages, p.exact_words, nullptr, 0, plan);
         int rc = V1_LAUNCHED("score_prep");
         if (rc != V1_OK) return rc;
         launch_hb<Shared>(hb, a->relu != 0, dim3((uint32_t)std::min<int64_t>(items, wgs)), st, p);
@@ -2116,7 +2160,7 @@ extern "C" int v1_score(const v1_score_args* a, void* stream) {
         // (records of the weights alone: the union form takes ReLU directly)
         hipLaunchKernelGGL(score_prep, row_waves, dim3(256), 0, st, a->q, a->weights, a->rows, a->heads,
                            a->relu ? 2 : 0, ws, p.work, p.exact_pages, p.exact_words,
-                           reinterpret_cast<uint32_t*>(u.level_n), (int32_t)kUnionLevels);
+                           reinterpret_cast<uint32_t*>(u.level_n), (int32_t)kUnionLevels, RangePlan{});
         int rc = V1_LAUNCHED("score_prep");
         if (rc != V1_OK) return rc;
         const int32_t hslots = plan_slots((int32_t)(kQueriesPerGroup * cdiv(a->max_context_len, 64)));

@@ -17,7 +17,7 @@ import torch
 
 from conftest import pkg
 from oracle import v1 as O
-from test_gpu_kernels import H, T, assert_scores_close
+from test_gpu_kernels import H, T, assert_scores_close, assert_scores_rel
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +88,34 @@ def test_relu_zeros_exact_and_topk_on_fp64_scores(dev, shared, heads, live, sign
     ident = np.arange(-(-ctx // 64), dtype=np.int32)[None].repeat(rows, 0)
     TK.topk_transform_512_v2(out, T(lens, dev), T(ident, dev), slots, 64, None, raw)
     assert np.array_equal(H(raw), _top_fp64(ref, lens, 2048))
+
+
+@pytest.mark.parametrize("rows,heads,longest,capacity", [
+    (600, 32, 5003, 5003),     # fewer 16-page chunks than work-groups: 14 pages
+    (9, 64, 1100, 16384),      # two groups, 4-page chunks, most of them past every row
+    (1030, 64, 8064, 16384),   # ranges of two chunks by the longest context, not by the capacity
+    (2000, 17, 8000, 8000),    # ranges of three chunks and a halving tail
+    (520, 16, 70, 40000),      # ranges of one chunk, all but the first empty
+    (40, 32, 0, 300),          # no row has a key
+])
+def test_shared_table_ranges(dev, rows, heads, longest, capacity):
+    """Shared-table scores over the ranges that the longest context and the
+    count of work-groups give, against the row-by-row kernel (each row its own
+    copy of the table, at most 512 rows a call).  4 live heads put keys on the
+    zero plateau, so marked pages cross the ranges too."""
+    g = np.random.default_rng(rows + heads)
+    live = 4
+    pages = -(-max(longest, 64) // 64)
+    q8, w, native, table = _probe_case(g, rows, heads, live, pages * 64, pages, False)[:4]
+    lens = g.integers(0, longest + 1, rows).astype(np.int32)
+    lens[rows // 2] = longest
+    tq, tn, tw, tl = T(q8, dev).view(torch.float8_e4m3fn), T(native, dev), T(w, dev), T(lens, dev)
+    tt = T(table, dev)[None]
+    out = torch.full((rows, capacity), 7.0, device=dev)
+    ref = torch.full((rows, capacity), 7.0, device=dev)
+    SC.fp8_paged_mqa_logits(tq, tn, tw, tl, tt.expand(rows, -1), None, capacity, clean_logits=True, out=out)
+    for r in range(0, rows, 512):
+        n = min(512, rows - r)
+        SC.fp8_paged_mqa_logits(tq[r:r + n], tn, tw[r:r + n], tl[r:r + n], tt.expand(n, -1).contiguous(), None, capacity,
+                                clean_logits=True, out=ref[r:r + n])
+    assert_scores_rel(H(out).astype(np.float64), H(ref).astype(np.float64))
