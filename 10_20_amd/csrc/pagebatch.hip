@@ -53,6 +53,74 @@ constexpr int kAggSlots = 2048;    // their LDS hash slots (>= 2 x kAggThreads, 
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+constexpr int kScanThreads = 1024;
+constexpr int kScanSteps = 8;      // runs of kScanThreads x 8 values
+constexpr int64_t kScanMax = (int64_t)kScanThreads * 8 * kScanSteps;  // values that one work-group scans
+
+// Exclusive prefix sums of n <= kScanMax values by one work-group of
+// kScanThreads; the sum of all is returned to every thread.  `in` and `out`
+// are 32-byte aligned and readable and writable to a multiple of 8 values.
+// All loads are in flight at once, so it takes about two memory round trips,
+// 6 us for 33 K values.  Past kScanMax the three launches of scan_exclusive
+// (4-5 us each, whatever the size) share the work better.  Sums, their
+// neighbours of one wave and the count's update in 13 launches for an insert
+// and a release instead of 20: 33 K entries of 42 KB 477 -> 457 us, of 8 KB
+// 142 -> 120, 200 entries 72 -> 49.
+__device__ uint32_t group_scan(const uint32_t* in, uint32_t* out, int32_t n) {
+    constexpr int kWaves = kScanThreads / kWave, kParts = kScanSteps * kWaves;
+    static_assert(kParts == 2 * kWave, "two partial sums per lane");
+    __shared__ uint32_t part[kParts];
+    __shared__ uint32_t all;
+    const int t = threadIdx.x, l = __lane_id(), w = t / kWave;
+    uint4 v[kScanSteps][2];
+#pragma unroll
+    for (int k = 0; k < kScanSteps; ++k) {
+        const int32_t i = (k * kScanThreads + t) * 8;
+        v[k][0] = v[k][1] = make_uint4(0u, 0u, 0u, 0u);
+        if (i < n) {
+            v[k][0] = reinterpret_cast<const uint4*>(in + i)[0];
+            v[k][1] = reinterpret_cast<const uint4*>(in + i)[1];
+        }
+    }
+    uint32_t mine[kScanSteps];
+#pragma unroll
+    for (int k = 0; k < kScanSteps; ++k) {
+        const int32_t left = n - (k * kScanThreads + t) * 8;  // values of this thread's eight
+        uint32_t* x = reinterpret_cast<uint32_t*>(v[k]);
+        uint32_t sum = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t here = i < left ? x[i] : 0u;
+            x[i] = sum;
+            sum += here;
+        }
+        const uint32_t incl = wave_inclusive_sum(sum);
+        mine[k] = incl - sum;
+        if (l == kWave - 1) part[k * kWaves + w] = incl;
+    }
+    __syncthreads();
+    if (w == 0) {
+        const uint32_t a = part[2 * l], b = part[2 * l + 1];
+        const uint32_t incl = wave_inclusive_sum(a + b);
+        part[2 * l] = incl - a - b;
+        part[2 * l + 1] = incl - b;
+        if (l == kWave - 1) all = incl;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kScanSteps; ++k) {
+        const int32_t i = (k * kScanThreads + t) * 8;
+        if (i >= n) continue;
+        const uint32_t base = part[k * kWaves + w] + mine[k];
+        uint4 a = v[k][0], b = v[k][1];
+        a.x += base, a.y += base, a.z += base, a.w += base;
+        b.x += base, b.y += base, b.z += base, b.w += base;
+        reinterpret_cast<uint4*>(out + i)[0] = a;
+        reinterpret_cast<uint4*>(out + i)[1] = b;
+    }
+    return all;
+}
+
 struct InsertState {
     uint8_t* pool;        // [cap, page_bytes]
     int64_t* pool_keys;   // [cap]
@@ -279,10 +347,16 @@ __global__ __launch_bounds__(kThreads) void pb_slow_live(InsertState s) {
     if (__lane_id() == 0) s.slow_live[k] = found;
 }
 
+__device__ __forceinline__ void wave_order() {  // one wave's memory accesses before and after, in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 // The colliding entries without an equal live page, one wave, in entry order:
 // the class of the earliest such entry with equal key and bytes, else a class
 // of its own.
-__global__ __launch_bounds__(kWave) void pb_slow(InsertState s) {
+__device__ void slow_entries(const InsertState& s) {
     __shared__ int32_t list[kSlowMax];
     __shared__ int32_t list_live[kSlowMax];
     __shared__ int32_t list_cls[kSlowMax];
@@ -295,7 +369,7 @@ __global__ __launch_bounds__(kWave) void pb_slow(InsertState s) {
     }
     // order by entry (distinct values): rank = number of smaller entries
     for (uint32_t k = l; k < ns; k += kWave) list_cls[k] = s.slow[k];
-    __syncthreads();
+    wave_order();
     for (uint32_t k = l; k < ns; k += kWave) {
         const int32_t e = list_cls[k];
         uint32_t r = 0;
@@ -303,7 +377,7 @@ __global__ __launch_bounds__(kWave) void pb_slow(InsertState s) {
         list[r] = e;
         list_live[r] = s.slow_live[k];
     }
-    __syncthreads();
+    wave_order();
     for (uint32_t k = 0; k < ns; ++k) {
         const int32_t e = list[k];
         int32_t c = list_live[k] >= 0 ? (list_live[k] | kClassLive) : -1;
@@ -319,8 +393,18 @@ __global__ __launch_bounds__(kWave) void pb_slow(InsertState s) {
             s.cls[e] = c;
             s.fresh[e] = fr;
         }
-        __syncthreads();
+        wave_order();
     }
+}
+
+__global__ __launch_bounds__(kWave) void pb_slow(InsertState s) { slow_entries(s); }
+
+// pb_slow and the fresh ranks in one launch (n <= kScanMax)
+__global__ __launch_bounds__(kScanThreads) void pb_slow_rank(InsertState s) {
+    if (threadIdx.x < kWave) slow_entries(s);
+    __syncthreads();
+    const uint32_t total = group_scan(s.fresh, s.rank, s.n);
+    if (threadIdx.x == 0) *s.nfresh = total;
 }
 
 // fresh pages from the free stack; the lowest fresh page of every batch class
@@ -374,10 +458,12 @@ __global__ __launch_bounds__(kAggThreads) void pb_table(InsertState s) {
         if (ids[t] >= 0) atomicAdd(&s.refs[ids[t]], cnt[t]);
 }
 
-// fresh pages receive the entry's bytes and key; work-groups stride over ranks
+// fresh pages receive the entry's bytes and key, work-groups striding over
+// ranks, and leave the free stack (nothing after pb_allocate reads its count)
 __global__ __launch_bounds__(kThreads) void pb_publish(InsertState s) {
     if (*s.abort) return;
     const uint32_t need = *s.nfresh;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *s.count -= (int32_t)need;
     const int64_t chunks = s.page_bytes >> 4;
     for (uint32_t r = blockIdx.x; r < need; r += gridDim.x) {
         const int32_t e = s.fresh_list[r];
@@ -400,10 +486,6 @@ __global__ __launch_bounds__(kThreads) void pb_publish(InsertState s) {
     }
 }
 
-__global__ void pb_commit(InsertState s) {
-    if (threadIdx.x == 0 && !*s.abort) *s.count -= (int32_t)*s.nfresh;
-}
-
 // ---------------------------------------------------------------- release
 struct ReleaseState {
     const int32_t* pages;  // [n] release order
@@ -418,6 +500,7 @@ struct ReleaseState {
     uint32_t* dead;    // [n]
     uint32_t* drank;   // [n]
     uint32_t* ndead;
+    int32_t* base;     // the free stack's count before the release
     uint32_t* abort;
 };
 
@@ -482,22 +565,35 @@ __global__ __launch_bounds__(kThreads) void rl_dead(ReleaseState s) {
     s.dead[i] = d;
 }
 
-__global__ __launch_bounds__(kThreads) void rl_commit(ReleaseState s) {
-    const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+// The free stack grows by the dead pages, or the release fails, before
+// rl_commit fills the new slots.
+__device__ void take_slots(const ReleaseState& s, uint32_t ndead) {
     if (*s.abort) return;
     const int32_t count = *s.count;
-    if (count < 0 || (int64_t)count + *s.ndead > s.cap) {  // more dead pages than free slots
-        if (i == 0) rfail(s, V1_STATUS_BAD_STATE);
+    if (count < 0 || (int64_t)count + ndead > s.cap) {  // more dead pages than free slots
+        rfail(s, V1_STATUS_BAD_STATE);
         return;
     }
-    if (i >= s.n) return;
-    const int32_t p = s.pages[i];
-    if (s.dead[i]) s.free_stack[count + (int32_t)s.drank[i]] = p;
-    if (s.last[p] == i) s.refs[p] -= s.cnt[p];
+    *s.base = count;
+    *s.count = count + (int32_t)ndead;
 }
 
-__global__ void rl_finish(ReleaseState s) {
-    if (threadIdx.x == 0 && !*s.abort) *s.count += (int32_t)*s.ndead;
+__global__ __launch_bounds__(kWave) void rl_take(ReleaseState s) {
+    if (threadIdx.x == 0) take_slots(s, *s.ndead);
+}
+
+// the dead pages' ranks and rl_take in one launch (n <= kScanMax)
+__global__ __launch_bounds__(kScanThreads) void rl_rank_take(ReleaseState s) {
+    const uint32_t ndead = group_scan(s.dead, s.drank, s.n);
+    if (threadIdx.x == 0) take_slots(s, ndead);
+}
+
+__global__ __launch_bounds__(kThreads) void rl_commit(ReleaseState s) {
+    const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (*s.abort || i >= s.n) return;
+    const int32_t p = s.pages[i];
+    if (s.dead[i]) s.free_stack[*s.base + (int32_t)s.drank[i]] = p;
+    if (s.last[p] == i) s.refs[p] -= s.cnt[p];
 }
 
 int64_t align256(int64_t x) { return (x + 255) & ~int64_t(255); }
@@ -547,7 +643,7 @@ InsertLayout insert_layout(int64_t cap, int64_t n) {
 }
 
 struct ReleaseLayout {
-    int64_t cnt, last, dead, drank, ndead, abort, scan_ws, total;
+    int64_t cnt, last, dead, drank, ndead, base, abort, scan_ws, total;
 };
 
 ReleaseLayout release_layout(int64_t cap, int64_t n) {
@@ -558,6 +654,7 @@ ReleaseLayout release_layout(int64_t cap, int64_t n) {
     L.dead = c.take(n * 4);
     L.drank = c.take(n * 4);
     L.ndead = c.take(4);
+    L.base = c.take(4);
     L.abort = c.take(4);
     L.scan_ws = c.take(scan_workspace(n));
     L.total = c.at;
@@ -623,14 +720,17 @@ extern "C" int v1_page_insert(uint8_t* pool, int64_t* pool_keys, int32_t* refs, 
     V1_CHECKED(name, hipLaunchKernelGGL(pb_classify, dim3((uint32_t)cdiv(n, kThreads / kWave)), dim3(kThreads), 0,
                                         st, s));
     V1_CHECKED(name, hipLaunchKernelGGL(pb_slow_live, dim3(kSlowMax / (kThreads / kWave)), dim3(kThreads), 0, st, s));
-    V1_CHECKED(name, hipLaunchKernelGGL(pb_slow, dim3(1), dim3(kWave), 0, st, s));
-    V1_OK_OR_RETURN(scan_exclusive(s.fresh, s.rank, s.nfresh, n, at<uint8_t>(w, L.scan_ws), scan_workspace(n), st,
-                                   name));
+    if (n <= kScanMax) {
+        V1_CHECKED(name, hipLaunchKernelGGL(pb_slow_rank, dim3(1), dim3(kScanThreads), 0, st, s));
+    } else {
+        V1_CHECKED(name, hipLaunchKernelGGL(pb_slow, dim3(1), dim3(kWave), 0, st, s));
+        V1_OK_OR_RETURN(scan_exclusive(s.fresh, s.rank, s.nfresh, n, at<uint8_t>(w, L.scan_ws), scan_workspace(n), st,
+                                       name));
+    }
     V1_CHECKED(name, hipLaunchKernelGGL(pb_allocate, grid_for(n), dim3(kThreads), 0, st, s));
     V1_CHECKED(name, hipLaunchKernelGGL(pb_table, dim3((uint32_t)cdiv(n, kAggThreads)), dim3(kAggThreads), 0, st, s));
     const uint32_t pub_groups = (uint32_t)std::min<int64_t>(n, 8 * (int64_t)device_cus());
     V1_CHECKED(name, hipLaunchKernelGGL(pb_publish, dim3(pub_groups), dim3(kThreads), 0, st, s));
-    V1_CHECKED(name, hipLaunchKernelGGL(pb_commit, dim3(1), dim3(kWave), 0, st, s));
     return V1_OK;
 }
 
@@ -652,14 +752,18 @@ extern "C" int v1_page_release(const int32_t* pages, int32_t n, int32_t* refs, i
     void* w = workspace;
     ReleaseState s{pages, n, refs, free_stack, count, capacity, status, at<int32_t>(w, L.cnt),
                    at<int32_t>(w, L.last), at<uint32_t>(w, L.dead), at<uint32_t>(w, L.drank),
-                   at<uint32_t>(w, L.ndead), at<uint32_t>(w, L.abort)};
+                   at<uint32_t>(w, L.ndead), at<int32_t>(w, L.base), at<uint32_t>(w, L.abort)};
     hipStream_t st = as_stream(stream);
     V1_CHECKED(name, hipLaunchKernelGGL(rl_init, grid_for(capacity), dim3(kThreads), 0, st, s));
     V1_CHECKED(name, hipLaunchKernelGGL(rl_count, dim3((uint32_t)cdiv(n, kAggThreads)), dim3(kAggThreads), 0, st, s));
     V1_CHECKED(name, hipLaunchKernelGGL(rl_dead, grid_for(n), dim3(kThreads), 0, st, s));
-    V1_OK_OR_RETURN(scan_exclusive(s.dead, s.drank, s.ndead, n, at<uint8_t>(w, L.scan_ws), scan_workspace(n), st,
-                                   name));
+    if (n <= kScanMax) {
+        V1_CHECKED(name, hipLaunchKernelGGL(rl_rank_take, dim3(1), dim3(kScanThreads), 0, st, s));
+    } else {
+        V1_OK_OR_RETURN(scan_exclusive(s.dead, s.drank, s.ndead, n, at<uint8_t>(w, L.scan_ws), scan_workspace(n), st,
+                                       name));
+        V1_CHECKED(name, hipLaunchKernelGGL(rl_take, dim3(1), dim3(kWave), 0, st, s));
+    }
     V1_CHECKED(name, hipLaunchKernelGGL(rl_commit, grid_for(n), dim3(kThreads), 0, st, s));
-    V1_CHECKED(name, hipLaunchKernelGGL(rl_finish, dim3(1), dim3(kWave), 0, st, s));
     return V1_OK;
 }

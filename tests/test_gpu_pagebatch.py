@@ -123,6 +123,30 @@ def test_page_insert_then_release_vs_oracle(dev, seed, page_bytes, collide):
     assert p.status() == 0
 
 
+@pytest.mark.parametrize("n", [1, 9, 8192, 8199, 65536, 65537])
+def test_page_ranks_at_scan_sizes(dev, n):
+    """Fresh and dead ranks at the edges of the one-work-group prefix sum (runs
+    of 8 values a thread, 8192 a step, 65536 in all) and one entry past it."""
+    g = np.random.default_rng(n)
+    cap = n + 3
+    keys = g.integers(0, max(1, n // 2), n).astype(np.int64)
+    req = np.sort(g.integers(0, max(1, n // 20), n)).astype(np.int32)
+    tmp = np.repeat(keys[:, None].view(np.uint8), 2, axis=1).reshape(n, 16)
+    if n > 9:
+        tmp[n // 2] ^= 255  # one colliding entry
+    st = (np.zeros((cap, 16), np.uint8), np.zeros(cap, np.int64), np.zeros(cap, np.int32),
+          g.permutation(cap).astype(np.int32), cap)
+    p = make_pool(dev, *st)
+    t = H(p.insert(T(keys, dev), T(tmp, dev), T(req, dev)))
+    exp = O.page_insert_batch(*st, keys, tmp, req)
+    assert np.array_equal(t, exp[0])
+    assert_state(p, *exp[1:])
+    rel = g.permutation(t).astype(np.int32)
+    p.release(T(rel, dev))
+    assert_state(p, exp[1], exp[2], *O.page_release_batch(rel, exp[3], exp[4], exp[5]))
+    assert p.status() == 0
+
+
 def test_page_insert_collision_classes(dev):
     """One key, many byte contents across requests: the one-wave resolution of
     colliding entries against live pages and earlier entries."""
