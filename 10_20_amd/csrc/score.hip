@@ -485,12 +485,11 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
         }
     }
   // A work-group's first item is its own number, and further ones are drawn
-  // from the counter (which score_prep leaves at zero): where items are short,
-  // behind the current item's first page loads, so that neither the next item
-  // nor the work-group's end waits on an atomic alone.  Long ones are drawn
-  // when the current one is done: held from its start, they leave the
-  // work-groups less even (32K keys x 4096 rows 780 -> 801 us).
-  const bool ahead = !UNION && full == 1;
+  // from the counter (which score_prep leaves at zero) when the current one is
+  // done; where every item is some work-group's first, none is.  (Drawn behind
+  // the current item's first page loads, they leave the work-groups less even:
+  // 4096 rows x 32K keys 780 -> 801 us, 2500 rows of 32 heads x 2700 46 -> 55.)
+  const bool more = UNION || total_items > (int32_t)gridDim.x;
   if (t == 0) item_sh = (int32_t)blockIdx.x;
   for (;;) {
     // every wave has finished the previous item (its LDS is free)
@@ -615,7 +614,7 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
     };
     __syncthreads();  // page ids in LDS; every wave has read item_sh
     if (npages == 0) {
-        if (t == 0) item_sh = (int32_t)(gridDim.x + atomicAdd(p.work, 1u));
+        if (t == 0) item_sh = more ? (int32_t)(gridDim.x + atomicAdd(p.work, 1u)) : total_items;
         fill_rest(0);
         continue;
     }
@@ -650,8 +649,6 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
         for (int j = 0; j < 2 * kWin; ++j)
             issue(ring[j], j < npages ? __builtin_amdgcn_readfirstlane(pids[j]) : -1);
     }
-    uint32_t drawn = 0u;
-    if (ahead && t == 0) drawn = atomicAdd(p.work, 1u);
 
     // B fragment of key block kb: key kb*16 + l%16, chunks 2*(l/16) and +1;
     // plus the scale of key l
@@ -898,7 +895,6 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
     // loaded above are complete before the loop, so no wait for them is
     // placed inside it.  (It also covers the first pages.)
     __builtin_amdgcn_s_waitcnt(0);
-    if (ahead && t == 0) item_sh = (int32_t)(gridDim.x + drawn);
     V1_PAGE_BARRIER(0);
 #pragma unroll
     for (int q = 0; q < QPW; ++q)
@@ -956,7 +952,7 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
         }
     }
     V1_PAGE_BARRIER(0);  // the page buffers are reused by the next item
-    if (!ahead && t == 0) item_sh = (int32_t)(gridDim.x + atomicAdd(p.work, 1u));
+    if (t == 0) item_sh = more ? (int32_t)(gridDim.x + atomicAdd(p.work, 1u)) : total_items;
     fill_rest(npages);
     if constexpr (UNION) {
         // marked pages to the rows' page bitmaps, at each row's table slot
@@ -2058,7 +2054,7 @@ extern "C" int v1_score(const v1_score_args* a, void* stream) {
         p.exact_words = fold ? exact_words(a->max_context_len) : 0;
         // Where even max_context_len gives a work-group fewer than two chunks,
         // ranges are one chunk and need no plan, nor its load before an item is
-        // known (1024 rows of 16 heads x 1024 keys 19.7 -> 16.5 us with 4-page
+        // known (1024 rows of 16 heads x 1024 keys 19.4 -> 14.8 us with 4-page
         // chunks, up to 22 us with a plan as well)
         p.planned = items / wgs > 1;
         const dim3 row_waves((uint32_t)cdiv(a->rows, 4)), prep_waves(row_waves.x + p.planned);
