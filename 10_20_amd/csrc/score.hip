@@ -70,8 +70,9 @@ struct ScoreParams {
     int32_t nchunks;        // shared-table kernel: chunks of chunk_pages pages over max_context_len
     int32_t chunk_pages;    // shared-table kernel: kChunkPages, or less where that leaves work-groups idle
     int32_t groups;         // shared-table kernel: 8-query row groups
-    int32_t planned;        // shared-table kernel: full ranges of work[1] chunks (else of one)
-    uint32_t* work;         // [0] next work item (zeroed by score_prep), [1] shared-table kernel: chunks of a full range
+    int32_t planned;        // shared-table kernel: work[2] and [3] hold a plan (else ranges of one chunk, all of them live)
+    uint32_t* work;         // [0] next work item (zeroed by score_prep); shared-table kernel: [2] chunks of a full range,
+                            // [3] chunks that the longest context reaches
     uint32_t* exact_pages;  // shared-table ReLU path: per row, a bitmap of pages for score_exact
     int32_t exact_words;    // 32-bit words per row of exact_pages (score_exact)
     // union form (per-row tables through the page ring), built by score_union_plan:
@@ -140,12 +141,17 @@ __device__ __forceinline__ float wave_all(float v, Op op) {
     return op(op(row(0), row(16)), op(row(32), row(48)));
 }
 
-// Chunks of a full range of score_shared's work items (work[1]), from the
-// longest context of the batch: about one range per work-group, at most
-// kMaxRange of them.  One range is one prologue, 6-7 us of dependent loads;
-// two half as long cost 2000 rows of 64 heads x 8000 keys 130 us against 114,
-// and a 1024-row query with 126 center pages 15 us more.  max_context_len in place of the longest
-// context would leave work-groups idle wherever it is a capacity and not a length.
+// Ranges of score_shared's work items, from the longest context of the batch:
+// the chunks that it reaches (work[3]) in about one full range per work-group
+// (work[2], at most max_range chunks).  One range is one prologue, 6-7 us of
+// dependent loads; two half as long cost 2000 rows of 64 heads x 8000 keys 130
+// us against 114, and a 1024-row query with 126 center pages 15 us more.
+// max_context_len in place of the longest context would leave work-groups idle
+// wherever it is a capacity and not a length.  The chunks past the longest
+// context hold no key: they are no score items at all, and with clean_logits
+// ranges that are only filled.  Cut like the others, they were empty items of a
+// prologue each: 4096 rows of 64 heads x 1024 keys in a capacity of 131072 took
+// 897 us (984 with clean_logits), now 47 (398; 2.1 GB of -inf).
 struct RangePlan {
     const int32_t* ctx;  // nullptr: no plan, no work-group for it
     int32_t max_context_len, chunk_pages, groups, wgs, max_range;
@@ -163,7 +169,8 @@ __device__ void plan_ranges(const RangePlan& plan, int32_t rows, uint32_t* work)
     longest = min(max(max(part[0], part[1]), max(part[2], part[3])), plan.max_context_len);
     const int64_t keys = 64 * (int64_t)plan.chunk_pages;
     const int64_t chunks = (longest + keys - 1) / keys;
-    work[1] = (uint32_t)max<int64_t>(1, min<int64_t>(plan.max_range, plan.groups * chunks / plan.wgs));
+    work[2] = (uint32_t)max<int64_t>(1, min<int64_t>(plan.max_range, plan.groups * chunks / plan.wgs));
+    work[3] = (uint32_t)chunks;
 }
 
 // One wave per query row: q' = sum_h w_h q_h split into its pieces, and the
@@ -418,6 +425,15 @@ constexpr int kUnionRange = 64;
 constexpr int kUnionLevels = 10;
 static_assert(kUnionRange == kWave && kUnionRange <= kMaxRangePages, "one union entry per lane");
 
+// Work items of a call (score_shared's own comment).
+struct ItemPlan {
+    int32_t full, bulk, live, live_items, fill, fills;
+};
+// Chunks of a fill range where a work-group gets several of them (one that it
+// gets alone may be twice that): 1024 rows x 4096 keys in a capacity of 131072
+// 119 us, 131 with 16.
+constexpr int kFillChunks = 8;
+
 // UNION: the item's pages are union entries of per-row tables (their columns
 // come from each row's table slot; a wave skips the MFMAs of a page none of
 // its queries lists, while the ring, the barriers and the store count go on
@@ -464,18 +480,40 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
     // union items per level (final before this kernel starts)
     int32_t lvl_n[UNION ? kUnionLevels : 1];
     // Shared tables: every group's ranges of `full` chunks first (`bulk` of
-    // them), then the rest of its chunks in ranges that halve in size, so that
-    // the last ones taken are short and the work-groups end together.
-    int32_t total_items, full = 0, bulk = 0;
-    auto range_chunks = [&](int32_t begin) __attribute__((always_inline)) {
-        return min((p.nchunks - begin + 1) / 2, full);
+    // them), then the rest of its live chunks in ranges that halve in size, so
+    // that the last ones taken are short and the work-groups end together.
+    // With clean_logits, ranges of `fill` chunks past the longest context are
+    // taken in turn with them, as long as there are both (stores beside
+    // products: 2048 rows of 32 heads x 8000 keys in a capacity of 65536 165
+    // -> 143 us).  In LDS: kept in registers, these counts cost the kernel of
+    // four head blocks its second work-group per CU.
+    __shared__ ItemPlan plan;
+    int32_t total_items;
+    auto range_chunks = [&](int32_t begin, int32_t live, int32_t full) __attribute__((always_inline)) {
+        return min((live - begin + 1) / 2, full);
     };
     if constexpr (!UNION) {
-        full = p.planned ? __builtin_amdgcn_readfirstlane((int32_t)p.work[1]) : 1;
-        bulk = p.nchunks > 2 * full ? __builtin_amdgcn_readfirstlane((p.nchunks - full) / full) : 0;
-        int32_t levels = bulk;
-        for (int32_t c = bulk * full; c < p.nchunks; c += range_chunks(c)) ++levels;
-        total_items = p.groups * levels;
+        ItemPlan x{};
+        x.full = 1;
+        x.live = p.nchunks;
+        if (p.planned) {
+            const int2 planned = *reinterpret_cast<const int2*>(p.work + 2);  // (one load: both are waited for)
+            x.full = __builtin_amdgcn_readfirstlane(planned.x);
+            x.live = __builtin_amdgcn_readfirstlane(planned.y);
+        }
+        x.bulk = x.live > 2 * x.full ? (x.live - x.full) / x.full : 0;
+        int32_t levels = x.bulk;
+        for (int32_t c = x.bulk * x.full; c < x.live; c += range_chunks(c, x.live, x.full)) ++levels;
+        x.live_items = p.groups * levels;
+        const int32_t wgs = gridDim.x, rest = p.clean ? p.nchunks - x.live : 0;
+        if (rest > 0) {
+            const int32_t takers = max(wgs - x.live_items, (wgs + 1) / 2);
+            x.fill = (p.groups * rest + takers - 1) / takers;
+            if (x.fill > 2 * kFillChunks) x.fill = kFillChunks;
+            x.fills = p.groups * ((rest + x.fill - 1) / x.fill);
+        }
+        total_items = x.live_items + x.fills;
+        if (t == 0) plan = x;
     } else {
         total_items = 0;
 #pragma unroll
@@ -494,8 +532,42 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
   for (;;) {
     // every wave has finished the previous item (its LDS is free)
     __syncthreads();
-    const int32_t item = __builtin_amdgcn_readfirstlane(item_sh);
+    int32_t item = __builtin_amdgcn_readfirstlane(item_sh);
     if (item >= total_items) break;
+    int32_t filled = -1;  // fill range, if the item is one
+    if constexpr (!UNION) {
+        const int32_t lives = __builtin_amdgcn_readfirstlane(plan.live_items);
+        const int32_t mixed = min(lives, __builtin_amdgcn_readfirstlane(plan.fills));
+        if (item < 2 * mixed) {
+            if (item & 1) filled = item >> 1;
+            else item >>= 1;
+        } else if (item >= mixed + lives) {
+            filled = item - lives;
+        } else {
+            item -= mixed;
+        }
+    }
+    if (!UNION && filled >= 0) {
+        __syncthreads();  // every wave has read item_sh
+        if (t == 0) item_sh = more ? (int32_t)(gridDim.x + atomicAdd(p.work, 1u)) : total_items;
+        const int32_t fill = plan.fill, begin = plan.live + filled / p.groups * fill;
+        const int32_t col = begin * p.chunk_pages * 64;
+        const uint32_t end = (uint32_t)min(begin + fill, p.nchunks) * p.chunk_pages * 64;  // (may pass 2^31)
+        const int32_t n = (int32_t)min(end, (uint32_t)p.max_context_len) - col;
+        const int64_t row = (int64_t)(filled % p.groups) * kQueriesPerGroup + wv * QPW;
+        int lane = l;
+        float x = -__builtin_huge_valf();
+        asm volatile("" : "+v"(lane), "+v"(x));  // keeps what follows from them inside the loop
+#pragma unroll 1
+        for (int q = 0; q < QPW; ++q) {
+            if (row + q >= p.rows) break;
+            float* const out = p.logits + (row + q) * p.logits_stride + col;
+            const int32_t quads = (reinterpret_cast<uintptr_t>(out) & 15) == 0 ? n >> 2 : 0;
+            for (int32_t i = lane; i < quads; i += kWave) reinterpret_cast<float4*>(out)[i] = make_float4(x, x, x, x);
+            for (int32_t i = 4 * quads + lane; i < n; i += kWave) out[i] = x;
+        }
+        continue;
+    }
     int32_t group, page_begin, nchunk = 0, ulen = 0;
     int64_t ubase = 0;  // union: the item's first entry
     if constexpr (UNION) {
@@ -513,12 +585,13 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
         ubase = (int64_t)group * p.u_cap + page_begin;
     } else {
         group = item % p.groups;
-        const int32_t level = item / p.groups;
+        const int32_t level = item / p.groups, full = __builtin_amdgcn_readfirstlane(plan.full);
+        const int32_t bulk = __builtin_amdgcn_readfirstlane(plan.bulk), live = __builtin_amdgcn_readfirstlane(plan.live);
         int32_t c_begin = min(level, bulk) * full;
-        nchunk = level < bulk ? full : range_chunks(c_begin);
+        nchunk = level < bulk ? full : range_chunks(c_begin, live, full);
         for (int32_t k = bulk; k < level; ++k) {
             c_begin += nchunk;
-            nchunk = range_chunks(c_begin);
+            nchunk = range_chunks(c_begin, live, full);
         }
         page_begin = c_begin * p.chunk_pages;
     }

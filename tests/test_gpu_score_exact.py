@@ -11,6 +11,8 @@ rows of ~2100 keys so that the Top-2048 boundary falls inside the plateau.
 Both the shared-table kernel (one page table for the whole chunk) and the
 per-row kernel are checked, and the selected indices are compared with a
 Top-2048 over the fp64 reference scores themselves."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -119,3 +121,47 @@ def test_shared_table_ranges(dev, rows, heads, longest, capacity):
         SC.fp8_paged_mqa_logits(tq[r:r + n], tn, tw[r:r + n], tl[r:r + n], tt.expand(n, -1).contiguous(), None, capacity,
                                 clean_logits=True, out=ref[r:r + n])
     assert_scores_rel(H(out).astype(np.float64), H(ref).astype(np.float64))
+
+
+@pytest.mark.parametrize("clean", [False, True])
+@pytest.mark.parametrize("rows,heads,longest,capacity", [
+    (4096, 16, 1024, 131072),   # one live chunk of 128
+    (1024, 32, 4096, 131072),
+    (259, 64, 500, 131000),     # ranges of one chunk, a last row group of three, a last page of 56 columns
+    (520, 64, 0, 33001),        # no live chunk, rows off 16-byte alignment
+])
+def test_shared_table_capacity_past_the_longest_context(dev, rows, heads, longest, capacity, clean):
+    """A capacity far above every context: the work items that work-groups draw
+    follow the longest context (the drawn count is the first word behind the
+    rows' records in the workspace), and the columns past it are -inf with
+    clean_logits and left alone without it."""
+    L = pkg("_lib")
+    g = np.random.default_rng(rows + longest)
+    pages = -(-max(longest, 64) // 64)
+    q8, w, native, table = _probe_case(g, rows, heads, 4, pages * 64, pages, False)[:4]
+    lens = g.integers(0, longest + 1, rows).astype(np.int32)
+    lens[rows // 2] = longest
+    tq, tn, tw, tl = T(q8, dev).view(torch.float8_e4m3fn), T(native, dev), T(w, dev), T(lens, dev)
+    tt = T(np.pad(table, (0, -(-capacity // 64) - pages)), dev)
+    lib = L.lib()
+    ws = torch.empty(lib.v1_score_workspace(rows, capacity), device=dev, dtype=torch.uint8)
+
+    def run(cap):
+        out = torch.full((rows, cap), 7.0, device=dev)
+        a = L.ScoreArgs(tq.data_ptr(), tn.data_ptr(), tn.shape[0], tw.data_ptr(), tl.data_ptr(), tt.data_ptr(), 0,
+                        tt.numel(), out.data_ptr(), out.stride(0), cap, rows, heads, 1, int(clean), ws.data_ptr(),
+                        ws.numel())
+        L.call("v1_score", ctypes.byref(a), torch.cuda.current_stream().cuda_stream)
+        at = lib.v1_score_workspace(rows, 0) - 256
+        return out, int(ws[at:at + 4].view(torch.int32).item())
+
+    out, drawn = run(capacity)
+    groups, chunks = -(-rows // 8), -(-longest // 1024)
+    work_groups = 2 * torch.cuda.get_device_properties(dev).multi_processor_count
+    filled = groups * (capacity // 8192 + 1) + work_groups if clean else 0  # (ranges of 8 chunks, or one a work-group)
+    assert drawn <= groups * chunks + filled + work_groups  # (each work-group's last draw finds none)
+    tight = run(max(longest, 1))[0]
+    assert_scores_rel(H(out[:, :longest]).astype(np.float64), H(tight[:, :longest]).astype(np.float64))
+    at = torch.arange(capacity, device=dev)[None] >= tl[:, None]
+    assert (out[at] == (-np.inf if clean else 7.0)).all()
+    assert torch.isfinite(out[~at]).all()
