@@ -14,6 +14,8 @@ twice by one row, entries that are -1 or past the pool (their keys read as
 zeros and score 0, as the per-row kernel gives), and groups that share too
 little (scored row by row).  The reference maps every invalid entry and every
 slot past the table to an all-zero page appended to the pool."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -344,3 +346,40 @@ def test_page_major_pair_table_sizes_and_repeats(dev, rows, pool_pages, blocks):
     finally:
         SC.page_major(prev)
     assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,listed,pool_pages", [(513, 80, 32000), (600, 1, 5000), (520, 41, 130)])
+def test_page_major_sparse_pool_touches_listed_chunks_alone(dev, rows, listed, pool_pages):
+    """Over a pool of which the rows list few pages, the pair table (the last
+    part of the workspace, 32 bytes per row and 8 listed pages) is written for
+    the listed pages' chunks and no others, and the scores are the bits of the
+    page-union plan."""
+    L = pkg("_lib")
+    g = np.random.default_rng(rows + listed)
+    heads, blocks = 20, 40
+    q8, w = _queries(g, rows, heads, heads)
+    k8, ks = W.quantize_rows(g.standard_normal((listed * 64, 128), dtype=np.float32))
+    where = g.permutation(pool_pages)[:listed]
+    native = torch.zeros((pool_pages, 8448), device=dev, dtype=torch.uint8)
+    native[T(where.astype(np.int64), dev)] = T(W.pack_pages(k8, ks), dev)
+    table = T(where[g.random((rows, max(listed, blocks))).argsort(1)[:, :blocks] % listed].astype(np.int32), dev)
+    table[0, :min(listed, blocks)] = T(where[:min(listed, blocks)].astype(np.int32), dev)
+    lens = g.integers(1, blocks * 64 + 1, rows).astype(np.int32)
+    tq, tw, tl = T(q8, dev).view(torch.float8_e4m3fn), T(w, dev), T(lens, dev)
+    used = len(np.unique(np.concatenate([H(table[r, :-(-int(n) // 64)]) for r, n in enumerate(lens)])))
+    width = blocks * 64
+    lib = L.lib()
+    ws = torch.full((lib.v1_score_pages_workspace(rows, width, pool_pages),), 0x5A, device=dev, dtype=torch.uint8)
+    out = torch.empty((rows, width), device=dev)
+    a = L.ScoreArgs(tq.data_ptr(), native.data_ptr(), pool_pages, tw.data_ptr(), tl.data_ptr(), table.data_ptr(),
+                    table.stride(0), blocks, out.data_ptr(), out.stride(0), width, rows, heads, 1, 1, ws.data_ptr(),
+                    ws.numel())
+    L.call("v1_score", ctypes.byref(a), torch.cuda.current_stream().cuda_stream)
+    pairs = ws[-(-(-pool_pages // 8) * rows * 32):].view(-1, rows * 32)
+    assert int((pairs != 0x5A).any(1).sum()) == -(-used // 8)
+    prev = SC.page_major(False)
+    try:
+        ref = SC.fp8_paged_mqa_logits(tq, native, tw, tl, table, None, width, clean_logits=True)
+    finally:
+        SC.page_major(prev)
+    assert torch.equal(out.view(torch.int32), ref.view(torch.int32))
