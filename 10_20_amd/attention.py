@@ -13,7 +13,7 @@ import math
 
 import torch
 
-from . import _lib, _workspace
+from . import _lib
 
 
 def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None, rotary_sin=None,
@@ -95,11 +95,17 @@ def attend_slots(q, k_pool, v_pool, request_slots, ids, head, softmax_scale=None
     elif out.dtype != torch.bfloat16 or tuple(out.shape) != (rows, 1, heads, 128) or out.stride(3) != 1:
         raise ValueError("out must be bfloat16 [rows, 1, heads, 128] with a contiguous head dimension")
     scale = float(softmax_scale) if softmax_scale is not None else 1.0 / math.sqrt(128)
-    ws, ws_bytes = _workspace.workspace(
-        q.device, _lib.lib().v1_decode_attention_slots_workspace(rows, heads, ids.shape[1]), "attend")
+    # The sums of a row's parts live from the call's first launch to its second.
+    # They are the call's own: another thread may launch on this stream between
+    # the two, and graphs captured on one stream may be replayed side by side.
+    # (The allocator hands the memory on in this stream's order, and a capture
+    # takes it from its own pool.)
+    ws_bytes = _lib.lib().v1_decode_attention_slots_workspace(rows, heads, ids.shape[1])
+    ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
     _lib.call("v1_decode_attention_slots_ws", _lib.ptr(q), q.stride(0), q.stride(1), _lib.ptr(k_pool), k_pool.stride(0),
               k_pool.stride(1), _lib.ptr(v_pool), v_pool.stride(0), v_pool.stride(1), k_pool.shape[0], int(head),
               _lib.ptr(request_slots), request_slots.numel(), _lib.ptr(ids), ids.stride(0), _lib.ptr(out),
-              out.stride(0), out.stride(2), rows, heads, ids.shape[1], scale, ws, ws_bytes, _lib.stream_of(q))
+              out.stride(0), out.stride(2), rows, heads, ids.shape[1], scale, _lib.ptr(ws), ws_bytes,
+              _lib.stream_of(q))
     return out
 
