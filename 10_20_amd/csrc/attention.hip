@@ -8,10 +8,10 @@
 // over the row's first n_b keys (n_b = seqlens[b] clamped to [0, S], or S);
 // a row with no keys gives zeros.
 //
-// One wave attends one part of a row's keys (parts as many as fill the GPU,
-// 1 from 2049 rows on, at most 16), tile by tile of 32 keys on the matrix
-// cores with a running maximum; the parts' sums are joined at the
-// end.  Both products are v_mfma_f32_16x16x32_bf16:
+// One wave attends one part of a row's keys (attn_parts: at most 8, 1 from 2049
+// rows on), tile by tile of 32 keys on the matrix cores with a running maximum;
+// the parts' sums are joined at the end.  Both products are
+// v_mfma_f32_16x16x32_bf16:
 //   scores  S^T = K Q^T: 16 keys x 16 columns, column n = head n % 4 (the same
 //           scores for n / 4 = 0 .. 3).  K goes memory -> LDS without passing
 //           registers (16-byte chunks of a 256-byte row XOR-swizzled by its
@@ -30,8 +30,11 @@
 // 256-byte pieces, 4.3 GB for 4096 rows of 2048 keys.  The form before this
 // one (16 lanes per key, fp32 products, two passes) spent ~130 vector
 // operations per 8 dims of a key and was bound by them: 717 us for those rows
-// over a context of 131072 slots, 4 heads; now 203-216 us (21 TB/s out of the
-// L2s; 1 head 519 -> 194 us), one row 97 -> 19 us.  Over rows of contiguous
+// over a context of 131072 slots, 4 heads; now 193-217 us (4.3 GB in that time
+// is 20-22 TB/s, which the L2s must give; 1 head 486 -> 190 us), one row 97 ->
+// 15 us, 1024 rows of 128 keys 18 -> 15 us.  One head of at most 96 keys alone
+// is slower than it was, by 0.1-0.5 us up to 1024 rows (4096 rows of 64 keys 23
+// -> 26 us): the prologue's and the join's latency.  Over rows of contiguous
 // keys (nothing shared) 822 -> 704 us, HBM's rate.
 //
 // Slot form: keys come straight from the K / V pools of one KV head through
@@ -53,8 +56,9 @@ constexpr int kMaxGroup = 4;       // heads of a P fragment: 16 rows / (3 parts,
 constexpr int kMaxScores = 12288;  // keys x heads that a call may have
 constexpr int kTile = 32;          // keys per step of a wave
 constexpr int kMaxWaves = 16;      // waves of a work-group
-constexpr int kMaxParts = 16;      // parts of a row's keys
 constexpr int kXcds = 8;
+constexpr int kMaxParts = kXcds;   // parts of a row's keys
+constexpr int kWaitAll = 0x0f70, kWaitButEight = 0x0f78;  // s_waitcnt vmcnt(0), vmcnt(8)
 
 // Lane p ^ J within 16-lane rows, every lane active.
 template <int J>
@@ -223,18 +227,11 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attn_kernel(AttnParams 
     int64_t b = blockIdx.y;
     bool extra = false;  // a wave past the last row: keeps the others' step, stores nothing
     if constexpr (LINED) {
-        // work-groups reach the XCDs in turn: each part's rows on 8 / parts of them (two parts on each at 16)
+        // work-groups reach the XCDs in turn: each part's rows on 8 / parts of them
         const int32_t rpb = (int32_t)blockDim.x / kWave, groups = (p.rows + rpb - 1) / rpb;
-        const int32_t xcd = (int32_t)(blockIdx.x % kXcds), i = (int32_t)(blockIdx.x / kXcds);
-        int32_t rg;
-        if (p.parts < kXcds) {
-            const int32_t per = kXcds / p.parts;
-            part = xcd / per;
-            rg = i * per + xcd % per;
-        } else {
-            part = xcd * (p.parts / kXcds) + i / groups;
-            rg = i % groups;
-        }
+        const int32_t xcd = (int32_t)(blockIdx.x % kXcds), i = (int32_t)(blockIdx.x / kXcds), per = kXcds / p.parts;
+        part = xcd / per;
+        const int32_t rg = i * per + xcd % per;
         if (rg >= groups) return;
         kvh = 0;
         b = (int64_t)rg * rpb + wave;
@@ -246,6 +243,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attn_kernel(AttnParams 
     // this wave's part of the row's tiles: `mine` of them from tile `first`
     const int32_t tiles = (n + kTile - 1) / kTile, each = (tiles + p.parts - 1) / p.parts;
     const int32_t first = min(part * each, tiles), mine = min(each, tiles - first);
+    const int32_t end = min((first + mine) * kTile, n);  // of its keys: what is fetched past them is the row of zeros
     WaveLds& my = wave_lds[wave];
 
     const char* kb = reinterpret_cast<const char*>(p.k + (SLOTS ? 0 : b * p.k_batch) + (int64_t)kvh * p.k_head);
@@ -258,10 +256,10 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attn_kernel(AttnParams 
     auto key_of = [&](int32_t it) __attribute__((always_inline)) { return (first + it) * kTile + (lane & 31); };
     auto fetch_id = [&](int32_t it) __attribute__((always_inline)) -> int32_t {
         if constexpr (!SLOTS) return 0;
-        else return p.ids[b * p.ids_stride + min(key_of(it), n - 1)];
+        else return p.ids[b * p.ids_stride + min(key_of(it), end - 1)];
     };
     auto id_ok = [&](int32_t it, int32_t id) __attribute__((always_inline)) -> int32_t {
-        return key_of(it) < n && (!SLOTS || (uint32_t)id < ids_end) ? -1 : 0;
+        return key_of(it) < end && (!SLOTS || (uint32_t)id < ids_end) ? -1 : 0;
     };
     auto fetch_slot = [&](int32_t id) __attribute__((always_inline)) -> int32_t {
         if constexpr (!SLOTS) return 0;
@@ -311,33 +309,42 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attn_kernel(AttnParams 
         __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(p.scale * 1.44269504088896341f)));
     const uint32_t cut1 = c >= 4 ? 0xffff0000u : 0u, cut2 = c >= 8 ? 0xffff0000u : 0u;
 
-    int32_t slot = 0, ok = 0, id = 0;  // slot and "id is in range" of tile it + 1, id of tile it + 2
-    if (mine > 0) {
-        id = fetch_id(0);
-        put_addr(0, id_ok(0, id), fetch_slot(id));
-        wave_lds_fence();
-        load_k();
-        asm volatile("" ::: "memory");
-        load_v();
-        id = fetch_id(1);
-        slot = fetch_slot(id);
-        ok = id_ok(1, id);
-        id = fetch_id(2);
-    }
     // B fragments of Q^T: column c = head c % 4 (those past the group repeat its last head, for nothing)
     Frag q[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s)
         q[s].u = *reinterpret_cast<const uint4*>(p.q + b * p.q_batch + (int64_t)(kvh * G + min(c & 3, G - 1)) * p.q_head +
                                                  32 * s + 8 * g);
-    // (landed before the loop, whose own waits count only its own loads)
+    // The first ids and slots are fetched side by side: a wave with one tile
+    // waits three times for memory (ids, slots, keys) before its first product.
+    int32_t slot = 0, ok = 0, id = 0;  // slot and "id is in range" of tile it + 1, id of tile it + 2
+    if (mine > 0) {
+        const int32_t id0 = fetch_id(0), id1 = fetch_id(1);
+        id = fetch_id(2);
+        const int32_t slot0 = fetch_slot(id0);
+        slot = fetch_slot(id1);
+        ok = id_ok(1, id1);
+        put_addr(0, id_ok(0, id0), slot0);
+        // (landed before the keys are fetched: the loop's own waits count only its own loads)
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-        asm volatile("" : "+v"(q[s].w[0]), "+v"(q[s].w[1]), "+v"(q[s].w[2]), "+v"(q[s].w[3]));
-    asm volatile("" : "+v"(slot), "+v"(id));
+        for (int s = 0; s < 4; ++s)
+            asm volatile("" : "+v"(q[s].w[0]), "+v"(q[s].w[1]), "+v"(q[s].w[2]), "+v"(q[s].w[3]));
+        asm volatile("" : "+v"(slot), "+v"(id)::"memory");
+        wave_lds_fence();
+        load_k();
+        asm volatile("" ::: "memory");
+        load_v();
+    }
 #pragma unroll 1
     for (int32_t it = 0; it < mine; ++it) {
         asm volatile("" : "+v"(k_chunk), "+v"(v_chunk), "+v"(k_read));  // (offsets made in place: kept, they spill)
+        // This tile's K, before ids and slots are fetched behind it (the wait
+        // that the compiler puts before the LDS reads would be for those too).
+        // Rows in step wait for V as well: it keeps them closer together (4096
+        // rows 197 us, 201 without; the other form 58-64 us for 64 rows, 66-80).
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(LINED ? kWaitAll : kWaitButEight);
+        asm volatile("" ::: "memory");
         put_addr(it + 1, ok, slot);  // this tile's addresses have been read
         slot = fetch_slot(id);
         ok = id_ok(it + 2, id);
@@ -345,7 +352,6 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attn_kernel(AttnParams 
         id = fetch_id(it + 3);
         // scores: rows r of MFMA group u are keys 8 (r / 4) + 4u + r % 4
         float s[8];
-        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // this tile's K (its V, issued after, may be on its way)
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             f32x4_t d = {0.f, 0.f, 0.f, 0.f};
@@ -360,9 +366,9 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attn_kernel(AttnParams 
             __builtin_amdgcn_sched_barrier(0);
         }
         wave_lds_fence();
-        load_k();
-        asm volatile("" ::: "memory");  // the next V loads stay behind: the wait above counts on it
-        const int32_t left = n - (first + it) * kTile - 8 * g;  // keys of this lane's eight
+        if (it + 1 < mine) load_k();
+        asm volatile("" ::: "memory");  // the next V loads stay behind: the next tile's wait counts on it
+        const int32_t left = end - (first + it) * kTile - 8 * g;  // keys of this lane's eight
 #pragma unroll
         for (int i = 0; i < 8; ++i) s[i] = i < left ? s[i] : -__builtin_inff();
         float top = s[0];
@@ -435,7 +441,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void decode_attn_kernel(AttnParams 
                 make_float4(acc[4][i], acc[5][i], acc[6][i], acc[7][i]);
         }
     } else {
-        plain_sums<SLOTS>(p, b, kb, vb, kvh, first * kTile, min(n, (first + mine) * kTile), sub, my);
+        plain_sums<SLOTS>(p, b, kb, vb, kvh, first * kTile, end, sub, my);
     }
     if constexpr (LINED) {
         wave_lds_fence();
@@ -492,14 +498,34 @@ __global__ __launch_bounds__(256) void join_kernel(AttnParams p) {
 }
 
 // Parts of a row's keys, a function of the call's (rows x KV heads) and keys
-// alone, so that every form adds the same sums in the same order: as many as
-// give each compute unit its 16 waves (4 per SIMD at 128 registers), at most
-// one per tile.
+// alone, so that every form adds the same sums in the same order: at most 8,
+// at most one per tile, and no more than give each SIMD two waves, or four
+// (what 128 registers allow) where each part keeps 8 tiles: a part costs a
+// prologue of three dependent loads and its share of the join. Measured, us:
+//   rows x keys      1      2      4      8     16 parts
+//     64 x 2048     64     36     22     19     20
+//    256 x  512     21     16     14     14     16
+//    512 x 2048     74     49     38     41     53
+//   1024 x  128     15     15     16
+//   2048 x 2048    114    110    120    137    178
+// (Up to 16 parts of one tile each, as many as four waves per SIMD, cost 1024
+// rows x 128 keys 27 us and 2048 rows x 64 28, more than the form before the
+// matrix cores.)
 inline int32_t attn_parts(int64_t groups, int32_t keys) {
-    const int64_t waves = (int64_t)kMaxWaves * device_cus(), tiles = cdiv(keys, kTile);
+    const int64_t waves = 8ll * device_cus(), tiles = cdiv(keys, kTile);
     int32_t parts = 1;
-    while (parts < kMaxParts && 2 * parts * groups <= waves && 2 * parts <= tiles) parts *= 2;
+    while (parts < kMaxParts && 2 * parts <= tiles &&
+           2 * parts * groups <= (tiles >= 16 * parts ? 2 * waves : waves))
+        parts *= 2;
     return parts;
+}
+
+// Parts in work-groups of their own, joined by a second launch, or the parts of
+// a row in one work-group: rows in step meet in the L2s, which pays for the
+// launch once the keys no longer fit them: 256 rows x 2048 keys 28 us, 38 in
+// one launch; 128 x 2048 24 / 25, 512 x 512 24 / 24, 256 x 128 10 / 6.
+inline bool attn_two_launches(int32_t rows, int32_t keys, int32_t parts) {
+    return parts > 1 && (int64_t)rows * keys > 1ll << 18;
 }
 
 inline int64_t attn_partial_bytes(int32_t rows, int32_t group, int32_t parts) {
@@ -525,7 +551,7 @@ inline int launch_lined(const AttnParams& p, hipStream_t st) {
     const int64_t rounds = cdiv(all, kMaxWaves * cus);
     const int32_t rpb = (int32_t)cdiv(all, rounds * cus);  // rows per work-group: one work-group per CU and round
     const int64_t groups = cdiv(p.rows, rpb);
-    const int64_t blocks = p.parts < kXcds ? kXcds * cdiv(groups, kXcds / p.parts) : groups * p.parts;
+    const int64_t blocks = kXcds * cdiv(groups, kXcds / p.parts);
     const int rc = launch_waves<true, true>(p, dim3((uint32_t)blocks), rpb, st);
     if (rc != V1_OK || p.parts == 1) return rc;
     hipLaunchKernelGGL(join_kernel, dim3((uint32_t)cdiv((int64_t)p.rows * p.group * kAttnDim, 256)), dim3(256), 0, st, p);
@@ -583,7 +609,8 @@ extern "C" int v1_decode_attention_slots_ws(const void* q, int64_t q_batch, int6
                  static_cast<uint16_t*>(out), o_batch, o_head, keys, heads_q, rows,
                  attn_parts(rows, keys), scale, ids, ids_stride, req, req_len, pool_slots, static_cast<float*>(workspace)};
     const int64_t need = attn_partial_bytes(rows, heads_q, p.parts);
-    if (p.parts == 1 || (workspace != nullptr && workspace_bytes >= need)) return launch_lined(p, as_stream(stream));
+    if (p.parts == 1 || (attn_two_launches(rows, keys, p.parts) && workspace != nullptr && workspace_bytes >= need))
+        return launch_lined(p, as_stream(stream));
     return launch_waves<true, false>(p, dim3(1, (uint32_t)rows), p.parts, as_stream(stream));
 }
 
@@ -601,5 +628,5 @@ extern "C" int v1_decode_attention_slots(const void* q, int64_t q_batch, int64_t
 extern "C" int64_t v1_decode_attention_slots_workspace(int32_t rows, int32_t heads_q, int32_t keys) {
     if (rows <= 0 || heads_q <= 0 || heads_q > kMaxGroup || keys <= 0) return 0;
     const int32_t parts = attn_parts(rows, keys);
-    return parts > 1 ? attn_partial_bytes(rows, heads_q, parts) : 0;
+    return attn_two_launches(rows, keys, parts) ? attn_partial_bytes(rows, heads_q, parts) : 0;
 }

@@ -137,10 +137,13 @@ def _slots_without_workspace(q, kp, vp, req, ids, head, scale):
     return out
 
 
-# rows choose the parts of a row's keys (1 at 4100 and 2100, 2 at 1100, ... 16 from 256 down) and the rows of a
-# work-group; keys the edges of 32-key tiles and of parts (parts without a key among them)
+# rows and keys choose the parts of a row's keys (1 from 1100 rows of 64 keys on, 2 at 33 keys, 8 at 1 x 2048 and
+# 130 x 2048), the rows of a work-group, and one launch or (more than 2^18 keys in all: the last four) two; keys are the
+# edges of 32-key tiles and of parts (parts without a key among them)
 @pytest.mark.parametrize("rows,keys,heads", [(1, 1, 4), (1, 2048, 1), (3, 31, 2), (17, 33, 3), (130, 65, 4),
-                                             (257, 1000, 2), (600, 97, 4), (1100, 64, 1), (2100, 40, 4), (4100, 32, 3)])
+                                             (257, 1000, 2), (600, 97, 4), (1100, 64, 1), (2100, 40, 4), (4100, 32, 3),
+                                             (9, 290, 4), (512, 512, 2), (130, 2048, 4), (257, 1100, 3), (1100, 520, 1),
+                                             (2048, 513, 2)])
 def test_attend_slots_parts_and_tiles(rows, keys, heads):
     g = torch.Generator(device=DEV).manual_seed(rows + keys)
     slots = 5000
