@@ -535,12 +535,10 @@ inline int64_t attn_partial_bytes(int32_t rows, int32_t group, int32_t parts) {
 template <bool SLOTS, bool LINED>
 int launch_waves(const AttnParams& p, dim3 grid, int32_t waves, hipStream_t st) {
     const size_t lds = sizeof(WaveLds) * (size_t)waves;
-    if (lds > 64 * 1024) {
-        const int rc = hip_status(hipFuncSetAttribute(reinterpret_cast<const void*>(decode_attn_kernel<SLOTS, LINED>),
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
-                                  "decode_attention: LDS");
-        if (rc != V1_OK) return rc;
-    }
+    static OncePerDevice lds_once;  // (to the most that any call takes: a smaller value would cut another thread's)
+    const int rc = allow_lds(lds_once, reinterpret_cast<const void*>(decode_attn_kernel<SLOTS, LINED>),
+                             sizeof(WaveLds) * (LINED ? kMaxWaves : kMaxParts), "decode_attention: LDS");
+    if (rc != V1_OK) return rc;
     hipLaunchKernelGGL((decode_attn_kernel<SLOTS, LINED>), grid, dim3(64 * waves), lds, st, p);
     return V1_LAUNCHED("decode_attention");
 }

@@ -8,6 +8,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 #include "../../include/v1idx.h"
+#include "per_device.h"
 
 namespace v1 {
 
@@ -50,6 +51,17 @@ inline int device_cus() {
         cus[dev] = (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) ? n : 256;
     }
     return cus[dev];
+}
+
+// Lets `kernel` take up to `bytes` of dynamic LDS on the current device (a
+// launch with more than 64 KiB needs it; the attribute is the device's own, so
+// that one call per process leaves every other device without it).
+inline int allow_lds(OncePerDevice& once, const void* kernel, size_t bytes, const char* what) {
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess) dev = -1;
+    return once.run(dev, [&] {
+        return hip_status(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes), what);
+    });
 }
 
 // ---------------------------------------------------------------- device side

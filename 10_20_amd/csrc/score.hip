@@ -2193,14 +2193,10 @@ extern "C" int v1_score(const v1_score_args* a, void* stream) {
             rc = V1_LAUNCHED("score_pages_rank");
             if (rc != V1_OK) return rc;
         }
-        // (dynamic LDS past 64 KiB needs the attribute, set once per process)
-        static std::once_flag place_once;
-        static hipError_t place_err = hipSuccess;
-        std::call_once(place_once, [] {
-            place_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&score_pages_place),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, kPmMaxPool * 4);
-        });
-        if (place_err != hipSuccess) return hip_status(place_err, "score: hipFuncSetAttribute(score_pages_place)");
+        static OncePerDevice place_once;
+        rc = allow_lds(place_once, reinterpret_cast<const void*>(&score_pages_place), kPmMaxPool * 4,
+                       "score: LDS of score_pages_place");
+        if (rc != V1_OK) return rc;
         hipLaunchKernelGGL(score_pages_place, dim3((uint32_t)a->rows), dim3(256), (size_t)L.chunks * kPmPages * 4, st, p, m);
         rc = V1_LAUNCHED("score_pages_place");
         if (rc != V1_OK) return rc;
@@ -2243,14 +2239,10 @@ extern "C" int v1_score(const v1_score_args* a, void* stream) {
         int rc = V1_LAUNCHED("score_prep");
         if (rc != V1_OK) return rc;
         const int32_t hslots = plan_slots((int32_t)(kQueriesPerGroup * cdiv(a->max_context_len, 64)));
-        // (dynamic LDS past 64 KiB needs the attribute, set once per process)
-        static std::once_flag lds_once;
-        static hipError_t lds_err = hipSuccess;
-        std::call_once(lds_once, [] {
-            lds_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&score_union_plan),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, 8 * kUnionEntries);
-        });
-        if (lds_err != hipSuccess) return hip_status(lds_err, "score: hipFuncSetAttribute(score_union_plan)");
+        static OncePerDevice plan_once;
+        rc = allow_lds(plan_once, reinterpret_cast<const void*>(&score_union_plan), 8 * kUnionEntries,
+                       "score: LDS of score_union_plan");
+        if (rc != V1_OK) return rc;
         hipLaunchKernelGGL(score_union_plan, dim3((uint32_t)groups), dim3(kPlanThreads), 8 * (size_t)hslots, st, p, u,
                            hslots);
         rc = V1_LAUNCHED("score_union_plan");
