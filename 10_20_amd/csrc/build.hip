@@ -247,13 +247,20 @@ __global__ __launch_bounds__(128) void assemble_kernel(const uint8_t* __restrict
 }
 
 // ------------------------------------------------------------- fused
-// Orders this wave's LDS accesses across its lanes (a wave's LDS operations
-// complete in order; the wait and the empty barrier keep the compiler from
-// moving accesses across the point).
-__device__ __forceinline__ void wave_sync() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
-}
+constexpr int kQuarter = 256;  // tokens of a quarter bucket
+
+// A position's token (of the bucket) and its unit divisor between the launches,
+// in memory that the last one writes: a quarter's part is written by the
+// quarter's own work-group, after it has read it.
+struct Carry {
+    int32_t* tok;
+    float* m;
+    int64_t bucket;   // words from a bucket to the next
+    int32_t quarter;  // and from a quarter to the next
+    __device__ int64_t at(int64_t b, int32_t pos) const {
+        return b * bucket + pos / kQuarter * quarter + pos % kQuarter;
+    }
+};
 
 // FP8 bytes 2H and 2H+1 of a packed word, as fp32 (exact).
 template <bool H>
@@ -398,25 +405,24 @@ __device__ __forceinline__ void dot_keys(Acc4& acc, const float (&a)[8], const u
 // Thread = position in the group (the bucket, or a half of it in the order
 // that the launch before left).  Three dots against the group's anchors
 // (first member, b = argmin s0, a = argmin sb), score = dot_a - sb, and a
-// stable descending sort by (score, -position).  Leaves the order in perm and
-// the unit divisors, as float bits, in map.  64 registers: two groups of 1024
-// share a CU, one's sort beside the other's dots.
+// stable descending sort by (score, -position).  64 registers: two groups of
+// 1024 share a CU, one's sort beside the other's dots.
 template <int N>
 __global__ __launch_bounds__(N, 8) void build_top_kernel(const uint8_t* __restrict__ pool, int64_t pool_pages,
-                                                         const int32_t* __restrict__ tables,
-                                                         int32_t* __restrict__ perm, int32_t* __restrict__ map) {
+                                                         const int32_t* __restrict__ tables, Carry carry) {
     __shared__ TopSmem<N> sm;
     const int32_t p = threadIdx.x, lane = p & (kWave - 1);
     const int32_t wave = __builtin_amdgcn_readfirstlane(p / kWave);
-    const int64_t b = blockIdx.x / (kTokens / N), at = (int64_t)blockIdx.x * N + p;
+    const int64_t b = blockIdx.x / (kTokens / N);
+    const int64_t at = carry.at(b, (int32_t)(blockIdx.x % (kTokens / N)) * N + p);
 
-    const int32_t tok = N == kTokens ? p : perm[at];
+    const int32_t tok = N == kTokens ? p : carry.tok[at];
     const int64_t page = page_of(tables + b * 16, tok, pool_pages);
     uint32_t c[kWords];
     load_key(pool + page * V1_PAGE_BYTES + (tok % 64) * 128, c);
     // the token's scale, unit divisor and its reciprocal
     const float s = reinterpret_cast<const float*>(pool)[page * kPageWords + kScaleWord + tok % 64];
-    const float m = N == kTokens ? unit_norm(c, s) : __int_as_float(map[at]);
+    const float m = N == kTokens ? unit_norm(c, s) : carry.m[at];
     const float rm = 1.0f / m;
     const Recip r = unit_recip(s, m, rm);
     const bool all_short = __builtin_amdgcn_ballot_w64(!short_units(s)) == 0;
@@ -467,12 +473,11 @@ __global__ __launch_bounds__(N, 8) void build_top_kernel(const uint8_t* __restri
     const uint64_t key = bitonic_sort<N>(((uint64_t)score_key(score) << 32) | (0xffffffffu - (uint32_t)p), p, wave,
                                          sm.k, nb);
     const int32_t from = (int32_t)(0xffffffffu - (uint32_t)key);  // old position of the new member
-    perm[at] = sm.tok[from];
-    map[at] = __float_as_int(sm.m[from]);
+    carry.tok[at] = sm.tok[from];
+    carry.m[at] = sm.m[from];
 }
 
 // ---- groups of 256 to 16: a quarter of a bucket per work-group
-constexpr int kQuarter = 256;
 constexpr int kQuarterWaves = kQuarter / kWave;
 
 // Tokens are numbered by their first position in the quarter; a thread's
@@ -492,18 +497,79 @@ __device__ __forceinline__ void dot_units(Acc4& acc, const float (&a)[8], const 
     if constexpr (W + 1 < kWords) dot_units<W + 1>(acc, a, u);
 }
 
+// Outputs of position `at` of bucket b, whose member is `id` of the work-group's
+// keys and token `tok` of the bucket: perm, its row of the assembled pages, the
+// member map, and its part of a center.  key(t, j) is 16-byte chunk j of key t.
+template <class Key, class Scale>
+__device__ __forceinline__ void write_member(int64_t b, int32_t at, int32_t id, int32_t tok, int32_t start,
+                                             int32_t* perm_out, uint8_t* tmp_out, int32_t* map_out,
+                                             uint8_t* centers_out, Key key, Scale scale_of) {
+    perm_out[b * kTokens + at] = tok;
+    map_out[b * kTokens + at] = start + tok;
+    uint8_t* tp = tmp_out + (b * 16 + at / 64) * V1_PAGE_BYTES;
+    uint4* row = reinterpret_cast<uint4*>(tp + (at % 64) * 128);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) row[j] = key(id, j);
+    reinterpret_cast<float*>(tp)[kScaleWord + at % 64] = scale_of(id);
+    // center at / 8: lane r of the 8 members computes dims 16r .. 16r+15
+    const int32_t lane = __lane_id(), r = lane & 7;
+    float mean[16];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int32_t t = __builtin_amdgcn_ds_bpermute(((lane & ~7) + j) << 2, id);
+        const uint4 w4 = key(t, r);
+        const float sj = scale_of(t);
+        const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float x0 = (fp8_at<0>(words[q]) * sj), x1 = (fp8_at<1>(words[q]) * sj);
+            const float x2 = (fp8_at<2>(words[q]) * sj), x3 = (fp8_at<3>(words[q]) * sj);
+            if (j == 0) {
+                mean[4 * q] = x0;
+                mean[4 * q + 1] = x1;
+                mean[4 * q + 2] = x2;
+                mean[4 * q + 3] = x3;
+            } else {
+                mean[4 * q] = (mean[4 * q] + x0);
+                mean[4 * q + 1] = (mean[4 * q + 1] + x1);
+                mean[4 * q + 2] = (mean[4 * q + 2] + x2);
+                mean[4 * q + 3] = (mean[4 * q + 3] + x3);
+            }
+        }
+    }
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        mean[i] = (mean[i] * 0.125f);
+        amax = fmaxf(amax, fabsf(mean[i]));
+    }
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
+    const float scale = center_scale(amax);
+    const float inv = 1.0f / scale;  // (a power of two from 2^-22 to 2^120: the products are the quotients)
+    uint32_t packed[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        packed[q] = e4m3_code(mean[4 * q] * inv) | (e4m3_code(mean[4 * q + 1] * inv) << 8) |
+                    (e4m3_code(mean[4 * q + 2] * inv) << 16) |
+                    (e4m3_code(mean[4 * q + 3] * inv) << 24);
+    const int32_t center = at / 8;
+    uint8_t* cp = centers_out + (b * 2 + center / 64) * V1_PAGE_BYTES;
+    *reinterpret_cast<uint4*>(cp + (center % 64) * 128 + 16 * r) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+    if (r == 0) reinterpret_cast<float*>(cp)[kScaleWord + center % 64] = scale;
+}
+
 // Thread = position in the quarter; the levels as above.  A level makes its
 // token's unit vector from the key in LDS (moving 128 registers instead costs
 // more LDS time than that takes vector time: 740 against 527 us for 2048
 // buckets when both were tried) and holds it through three dots.  Groups of at most one wave run
-// without barriers.  Then the quarter's pages, member map, order and centers.
+// without barriers.  Then the outputs of the quarter, or (tmp_out null) its
+// order alone.
 __global__ __launch_bounds__(kQuarter, 3) void build_quarter_kernel(const uint8_t* __restrict__ pool, int64_t pool_pages,
                                                                     const int32_t* __restrict__ tables,
-                                                                    const int32_t* __restrict__ starts,
-                                                                    int32_t* __restrict__ perm_out,
-                                                                    uint8_t* __restrict__ tmp_out,
-                                                                    int32_t* __restrict__ map_out,
-                                                                    uint8_t* __restrict__ centers_out) {
+                                                                    const int32_t* __restrict__ starts, Carry carry,
+                                                                    int32_t* perm_out, uint8_t* tmp_out,
+                                                                    int32_t* map_out, uint8_t* centers_out) {
     __shared__ QuarterSmem sm;
     const int32_t p = threadIdx.x, lane = p & (kWave - 1);
     const int32_t wave = __builtin_amdgcn_readfirstlane(p / kWave);
@@ -513,8 +579,8 @@ __global__ __launch_bounds__(kQuarter, 3) void build_quarter_kernel(const uint8_
     int32_t id = p;
     bool all_short;
     {
-        const int32_t tok = perm_out[b * kTokens + at];
-        const float m = __int_as_float(map_out[b * kTokens + at]);
+        const int32_t tok = carry.tok[carry.at(b, at)];
+        const float m = carry.m[carry.at(b, at)];
         const int64_t page = page_of(tables + b * 16, tok, pool_pages);
         const uint4* src = reinterpret_cast<const uint4*>(pool + page * V1_PAGE_BYTES + (tok % 64) * 128);
 #pragma unroll
@@ -608,64 +674,38 @@ __global__ __launch_bounds__(kQuarter, 3) void build_quarter_kernel(const uint8_
     level(std::integral_constant<int32_t, 32>());
     level(std::integral_constant<int32_t, 16>());
 
-    // final order: perm, the assembled pages, member map and centers
-    const float4 v = sm.v[id];
-    const int32_t tok = __float_as_int(v.w);
-    perm_out[b * kTokens + at] = tok;
-    map_out[b * kTokens + at] = starts[b] + tok;
-    uint8_t* tp = tmp_out + (b * 16 + at / 64) * V1_PAGE_BYTES;
-    uint4* row = reinterpret_cast<uint4*>(tp + (at % 64) * 128);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) row[j] = sm.c[id][j ^ (id & 7)];
-    reinterpret_cast<float*>(tp)[kScaleWord + at % 64] = v.x;
-    // center at / 8: lane r of the 8 members computes dims 16r .. 16r+15
-    const int32_t r = p & 7;
-    float mean[16];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int32_t t = __builtin_amdgcn_ds_bpermute(((lane & ~7) + j) << 2, id);
-        const uint4 w4 = sm.c[t][r ^ (t & 7)];
-        const float sj = sm.v[t].x;
-        const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float x0 = (fp8_at<0>(words[q]) * sj), x1 = (fp8_at<1>(words[q]) * sj);
-            const float x2 = (fp8_at<2>(words[q]) * sj), x3 = (fp8_at<3>(words[q]) * sj);
-            if (j == 0) {
-                mean[4 * q] = x0;
-                mean[4 * q + 1] = x1;
-                mean[4 * q + 2] = x2;
-                mean[4 * q + 3] = x3;
-            } else {
-                mean[4 * q] = (mean[4 * q] + x0);
-                mean[4 * q + 1] = (mean[4 * q + 1] + x1);
-                mean[4 * q + 2] = (mean[4 * q + 2] + x2);
-                mean[4 * q + 3] = (mean[4 * q + 3] + x3);
-            }
-        }
+    const int32_t tok = __float_as_int(sm.v[id].w);
+    if (tmp_out == nullptr) {  // (build_write_kernel writes the outputs)
+        carry.tok[carry.at(b, at)] = tok;
+        return;
     }
-    float amax = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        mean[i] = (mean[i] * 0.125f);
-        amax = fmaxf(amax, fabsf(mean[i]));
-    }
-#pragma unroll
-    for (int off = 1; off < 8; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
-    const float scale = center_scale(amax);
-    const float inv = 1.0f / scale;  // (a power of two from 2^-22 to 2^120: the products are the quotients)
-    uint32_t packed[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        packed[q] = e4m3_code(mean[4 * q] * inv) | (e4m3_code(mean[4 * q + 1] * inv) << 8) |
-                    (e4m3_code(mean[4 * q + 2] * inv) << 16) |
-                    (e4m3_code(mean[4 * q + 3] * inv) << 24);
-    const int32_t center = at / 8;
-    uint8_t* cp = centers_out + (b * 2 + center / 64) * V1_PAGE_BYTES;
-    *reinterpret_cast<uint4*>(cp + (center % 64) * 128 + 16 * r) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-    if (r == 0) reinterpret_cast<float*>(cp)[kScaleWord + center % 64] = scale;
+    write_member(b, at, id, tok, starts[b], perm_out, tmp_out, map_out, centers_out,
+                 [&](int32_t t, int32_t j) __attribute__((always_inline)) { return sm.c[t][j ^ (t & 7)]; },
+                 [&](int32_t t) __attribute__((always_inline)) { return sm.v[t].x; });
 }
 
+// The outputs of a bucket in the order that the launches before left, by one
+// work-group that has read all of the bucket before it writes: for outputs that
+// lie over the bucket's own pages.
+__global__ __launch_bounds__(kTokens) void build_write_kernel(const uint8_t* pool, int64_t pool_pages,
+                                                              const int32_t* tables, const int32_t* starts, Carry carry,
+                                                              int32_t* perm_out, uint8_t* tmp_out, int32_t* map_out,
+                                                              uint8_t* centers_out) {
+    __shared__ uint4 c[kTokens][8];
+    __shared__ float s[kTokens];
+    const int32_t p = threadIdx.x;
+    const int64_t b = blockIdx.x;
+    const int32_t tok = carry.tok[carry.at(b, p)], start = starts[b];
+    const int64_t page = page_of(tables + b * 16, tok, pool_pages);
+    const uint4* src = reinterpret_cast<const uint4*>(pool + page * V1_PAGE_BYTES + (tok % 64) * 128);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) c[p][j ^ (p & 7)] = src[j];
+    s[p] = reinterpret_cast<const float*>(pool)[page * kPageWords + kScaleWord + tok % 64];
+    __syncthreads();
+    write_member(b, p, p, tok, start, perm_out, tmp_out, map_out, centers_out,
+                 [&](int32_t t, int32_t j) __attribute__((always_inline)) { return c[t][j ^ (t & 7)]; },
+                 [&](int32_t t) __attribute__((always_inline)) { return s[t]; });
+}
 
 }  // namespace
 }  // namespace v1
@@ -721,16 +761,40 @@ extern "C" int v1_build_buckets(const void* pool, int64_t pool_pages, const int3
                    (reinterpret_cast<uintptr_t>(centers) & 15) == 0,
                "build_buckets: pool, tmp and centers must be 16-byte aligned");
     if (buckets == 0) return V1_OK;
-    hipLaunchKernelGGL(build_top_kernel<1024>, dim3((uint32_t)buckets), dim3(1024), 0, as_stream(stream),
-                       static_cast<const uint8_t*>(pool), pool_pages, tables, perm, mapping);
+    // Outputs over a bucket's own pages are allowed (all of the bucket is read
+    // before any of them is written); quarters that read and write side by side
+    // are for outputs elsewhere.  The order between the launches lies in tmp, or
+    // in perm and mapping where tmp is over the pool.
+    const int64_t pool_bytes = pool_pages * V1_PAGE_BYTES, order_bytes = (int64_t)buckets * kTokens * 4;
+    auto meet = [](const void* a, int64_t na, const void* b, int64_t nb) {
+        const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+        return x < y + (uintptr_t)nb && y < x + (uintptr_t)na;
+    };
+    const bool tmp_meets = meet(pool, pool_bytes, tmp, (int64_t)buckets * 16 * V1_PAGE_BYTES);
+    const bool order_meets = meet(pool, pool_bytes, perm, order_bytes) || meet(pool, pool_bytes, mapping, order_bytes);
+    const bool in_place = tmp_meets || order_meets ||
+                          meet(pool, pool_bytes, centers, (int64_t)buckets * 2 * V1_PAGE_BYTES);
+    V1_REQUIRE(!tmp_meets || !(order_meets || meet(perm, order_bytes, mapping, order_bytes)),
+               "build_buckets: with tmp over the pool, perm and mapping must be apart from it and from each other");
+    Carry carry{perm, reinterpret_cast<float*>(mapping), kTokens, kQuarter};
+    if (!tmp_meets) {
+        carry = Carry{static_cast<int32_t*>(tmp), static_cast<float*>(tmp) + kQuarter, 16 * kPageWords, 4 * kPageWords};
+    }
+    const uint8_t* const from = static_cast<const uint8_t*>(pool);
+    uint8_t* const pages = static_cast<uint8_t*>(tmp);
+    uint8_t* const means = static_cast<uint8_t*>(centers);
+    hipStream_t st = as_stream(stream);
+    hipLaunchKernelGGL(build_top_kernel<1024>, dim3((uint32_t)buckets), dim3(1024), 0, st, from, pool_pages, tables, carry);
     int rc = V1_LAUNCHED("build_buckets: 1024");
     if (rc != V1_OK) return rc;
-    hipLaunchKernelGGL(build_top_kernel<512>, dim3((uint32_t)buckets * 2), dim3(512), 0, as_stream(stream),
-                       static_cast<const uint8_t*>(pool), pool_pages, tables, perm, mapping);
+    hipLaunchKernelGGL(build_top_kernel<512>, dim3((uint32_t)buckets * 2), dim3(512), 0, st, from, pool_pages, tables, carry);
     rc = V1_LAUNCHED("build_buckets: 512");
     if (rc != V1_OK) return rc;
-    hipLaunchKernelGGL(build_quarter_kernel, dim3((uint32_t)buckets * (kTokens / kQuarter)), dim3(kQuarter), 0,
-                       as_stream(stream), static_cast<const uint8_t*>(pool), pool_pages, tables, starts, perm,
-                       static_cast<uint8_t*>(tmp), mapping, static_cast<uint8_t*>(centers));
-    return V1_LAUNCHED("build_buckets: quarters");
+    hipLaunchKernelGGL(build_quarter_kernel, dim3((uint32_t)buckets * (kTokens / kQuarter)), dim3(kQuarter), 0, st, from,
+                       pool_pages, tables, starts, carry, perm, in_place ? nullptr : pages, mapping, means);
+    rc = V1_LAUNCHED("build_buckets: quarters");
+    if (rc != V1_OK || !in_place) return rc;
+    hipLaunchKernelGGL(build_write_kernel, dim3((uint32_t)buckets), dim3(kTokens), 0, st, from, pool_pages, tables, starts,
+                       carry, perm, pages, mapping, means);
+    return V1_LAUNCHED("build_buckets: outputs");
 }

@@ -354,11 +354,14 @@ int v1_build_assemble(const void* K, const float* KS, const int32_t* table, cons
                       int32_t pages, int32_t groups, void* stream);
 /* The chain initialize -> 7 x (3 _dots, 2 _anchor, _sort) -> assemble of
  * sglang/srt/layers/attention/v1_deepseek/runtime.py:171-216 for a batch of
- * buckets in one launch: bucket b reads pages tables[b*16 .. b*16+15] of the
+ * buckets in one call: bucket b reads pages tables[b*16 .. b*16+15] of the
  * pool and writes perm [b, 1024] (token order, 0..1023), tmp [b, 16 pages],
  * mapping [b, 1024] = starts[b] + perm and centers [b, 2 pages].  Identical
  * results to the chain of the entry points above.  Table entries outside
- * [0, pool_pages) read page 0. */
+ * [0, pool_pages) read page 0.  A bucket's outputs may lie over its own source
+ * pages (all of the bucket is read before any of them is written), not over
+ * another bucket's; with tmp over the pool, perm and mapping must lie apart
+ * from the pool and from each other (they hold the order meanwhile). */
 int v1_build_buckets(const void* pool, int64_t pool_pages, const int32_t* tables, const int32_t* starts,
                      int32_t buckets, int32_t* perm, void* tmp, int32_t* mapping, void* centers, void* stream);
 

@@ -214,3 +214,44 @@ def test_build_buckets_scales(mods, factors):
         e_perm, e_tmp, e_map, e_centers = O.index_build(pool, tables[b], int(starts[b]))
         assert np.array_equal(H(perm[b]), e_perm) and np.array_equal(H(tmp[b]), e_tmp)
         assert np.array_equal(H(mapping[b]), e_map) and np.array_equal(H(centers[b]), e_centers)
+
+
+@pytest.mark.parametrize("buckets", [1, 5])
+def test_build_buckets_in_place(mods, buckets):
+    """tmp over the buckets' own source pages (each bucket's pages sorted where
+    they lie), centers over the first two of them, mapping over perm: the bytes
+    of a call with outputs of their own."""
+    _, _, IB = mods
+    g = np.random.default_rng(buckets)
+    pool = T(np.concatenate([_pool(40 + i) for i in range(buckets)])[:16 * buckets])
+    tables = T(np.stack([16 * b + g.permutation(16) for b in range(buckets)]).astype(np.int32))
+    starts = T((1024 * np.arange(buckets)).astype(np.int32))
+    perm, tmp, mapping, centers = IB.build_buckets(pool, tables, starts)
+
+    def outs():
+        return [torch.full_like(x, 7) for x in (perm, tmp, mapping, centers)]
+
+    def check(got, skip=()):
+        for i, (x, y) in enumerate(zip(got, (perm, tmp, mapping, centers))):
+            assert i in skip or torch.equal(x.reshape(-1), y.reshape(-1)), i
+
+    p, o = pool.clone(), outs()
+    o[1] = p.view(buckets, 16, 8448)
+    check(IB.build_buckets(p, tables, starts, out=o))
+    o = outs()
+    o[0] = o[2].view(buckets, 1024)
+    check(IB.build_buckets(pool, tables, starts, out=o), skip=(0,))
+    if buckets == 1:
+        p, o = pool.clone(), outs()
+        o[3] = p[:2][None]
+        check(IB.build_buckets(p, tables, starts, out=o))
+        p, o = pool.clone(), outs()
+        o[0] = p[3:4, :4096].view(torch.int32)
+        o[2] = p[5:6, 4096:8192].view(torch.int32)
+        check(IB.build_buckets(p, tables, starts, out=o))
+    p, o = pool.clone(), outs()
+    o[1] = p.view(buckets, 16, 8448)
+    o[0] = o[2].view(buckets, 1024)
+    with pytest.raises(ValueError, match="apart"):
+        IB.build_buckets(p, tables, starts, out=o)
+    assert torch.equal(p, pool)
