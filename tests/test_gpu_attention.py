@@ -190,3 +190,77 @@ def test_attend_slots_infinite_values():
     assert math.isnan(got[2, 5]) and got[2, 0] == 1
     assert (got[3] == 1).all()
     assert np.isnan(got[4]).all()
+
+
+def _nonfinite_reference(q, k, v, n, scale):
+    """O[b, h] in fp64 over the first n[b] keys, a weight of zero (a masked key)
+    left out of the sum: q [B, H, 128], k / v [B, S, H, 128] expanded to the
+    query heads.  Also the bound of a finite output."""
+    s = torch.einsum("bhd,bshd->bhs", q.double().cpu(), k.double().cpu()) * scale
+    live = torch.arange(k.shape[1])[None, None] < n[:, None, None]
+    p = torch.softmax(s.masked_fill(~live, -math.inf), -1)
+    v = v.double().cpu()
+    ref = torch.zeros(q.shape, dtype=torch.float64)
+    mag = torch.zeros_like(ref)
+    for j in range(k.shape[1]):
+        w = p[:, :, j, None]
+        ref += torch.where(live[:, :, j, None], w * v[:, j], torch.zeros(()).double())
+        mag += torch.where(live[:, :, j, None], w * v[:, j].abs(), torch.zeros(()).double())
+    terms = torch.einsum("bhd,bshd->bhs", q.double().cpu().abs(), k.double().cpu().abs()).amax() * scale
+    return ref, ref.abs() * (2**-8 + 2**-16) + mag * (2 * terms * 2**-16 + 2**-13)
+
+
+def _check_nonfinite(got, ref, bound):
+    got = got.double().cpu()
+    assert torch.equal(got.isnan(), ref.isnan())
+    inf = ref.isinf()
+    assert torch.equal(got[inf], ref[inf])
+    fin = ref.isfinite()
+    assert ((got - ref).abs() <= bound)[fin].all()
+
+
+# infinite values in the first, a middle and the last tile of a row, of one sign and of both in one dim, met before and
+# after the running maximum rises (keys of `rising` rows score ever higher, of others ever lower); rows without any
+# beside them.  Scores lie within +-20: no weight underflows, whose product with an infinity would be NaN.
+@pytest.mark.parametrize("keys,heads,rows", [(33, 1, 3), (97, 2, 5), (97, 4, 700), (1000, 3, 9), (1000, 4, 300),
+                                             (260, 4, 1030)])
+@pytest.mark.parametrize("form", ["slots", "gathered"])
+def test_infinite_values_in_tiles_and_parts(keys, heads, rows, form):
+    g = torch.Generator(device=DEV).manual_seed(keys + heads)
+    kv_heads = 1 if form == "slots" else 2
+    k = 0.2 * torch.randn((rows, keys, kv_heads, 128), device=DEV, generator=g)
+    k[..., 0] = torch.linspace(-1, 1, keys, device=DEV)[None, :, None]
+    k[1::2, :, :, 0] *= -1
+    k = k.to(torch.bfloat16)
+    v = torch.randn((rows, keys, kv_heads, 128), device=DEV, generator=g).to(torch.bfloat16)
+    q = torch.randn((rows, heads * kv_heads, 128), device=DEV, generator=g)
+    q[..., 0] = 8
+    q = q.to(torch.bfloat16)
+    n = torch.full((rows,), keys)
+    if form == "gathered":
+        n[::3] = torch.arange(len(n[::3])) % keys + 1
+    for r in range(0, rows, 2 if rows < 20 else 37):
+        last = int(n[r]) - 1
+        v[r, 0, :, 1] = math.inf
+        v[r, last // 2, :, 2] = -math.inf
+        v[r, last, :, 3] = math.inf
+        v[r, 0, 0, 4], v[r, last, 0, 4] = math.inf, -math.inf
+        if last + 1 < keys:
+            v[r, last + 1:, :, 5] = math.inf  # past the row's length
+    scale = 1.0
+    if form == "gathered":
+        got = AT.flash_attn_with_kvcache(q[:, None], k, v, cache_seqlens=n.to(DEV, torch.int32), softmax_scale=scale)[:, 0]
+    else:
+        ids = torch.randperm(rows * keys, device=DEV, generator=g).view(rows, keys).to(torch.int32)
+        req = torch.empty(rows * keys, device=DEV, dtype=torch.int32)
+        req[ids.long().reshape(-1)] = torch.arange(rows * keys, device=DEV, dtype=torch.int32)
+        args = (q, k.reshape(rows * keys, 1, 128), v.reshape(rows * keys, 1, 128), req, ids, 0)
+        got = AT.attend_slots(*args, softmax_scale=scale)[:, 0]
+        one = _slots_without_workspace(*args, scale)[:, 0]
+        assert torch.equal(got.isnan(), one.isnan()) and torch.equal(got.nan_to_num(7.0), one.nan_to_num(7.0))
+    some = torch.arange(0, rows, 1 if rows < 20 else 37)
+    some = torch.unique(torch.cat([some, (some + 1).clamp_max(rows - 1)]))
+    ref, bound = _nonfinite_reference(q[some], k[some].repeat_interleave(heads, 2),
+                                      v[some].repeat_interleave(heads, 2), n[some], scale)
+    assert ref.isinf().any() and ref.isnan().any() and ref.isfinite().any()
+    _check_nonfinite(got[some], ref, bound)
