@@ -501,6 +501,9 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
             x.full = __builtin_amdgcn_readfirstlane(planned.x);
             x.live = __builtin_amdgcn_readfirstlane(planned.y);
         }
+        // (a remainder that ends a score range costs no item of its own: a
+        // 1024-row query with 126 of 136 center pages 455 -> 452 us)
+        if (p.clean && p.nchunks - x.live <= x.full) x.live = p.nchunks;
         x.bulk = x.live > 2 * x.full ? (x.live - x.full) / x.full : 0;
         int32_t levels = x.bulk;
         for (int32_t c = x.bulk * x.full; c < x.live; c += range_chunks(c, x.live, x.full)) ++levels;
