@@ -485,15 +485,17 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
     // With clean_logits, ranges of `fill` chunks past the longest context are
     // taken in turn with them, as long as there are both (stores beside
     // products: 2048 rows of 32 heads x 8000 keys in a capacity of 65536 165
-    // -> 143 us).  In LDS: kept in registers, these counts cost the kernel of
-    // four head blocks its second work-group per CU.
-    __shared__ ItemPlan plan;
+    // -> 143 us).  Kept in registers, these counts cost the kernel of four head
+    // blocks its second work-group per CU, which reads them from LDS; the others
+    // keep them (1024 rows of 16 heads x 1024 keys 13.9 us, 14.2 from LDS).
+    __shared__ ItemPlan plan_sh;
+    ItemPlan x{};
+    const ItemPlan& plan = HB == 4 ? plan_sh : x;
     int32_t total_items;
     auto range_chunks = [&](int32_t begin, int32_t live, int32_t full) __attribute__((always_inline)) {
         return min((live - begin + 1) / 2, full);
     };
     if constexpr (!UNION) {
-        ItemPlan x{};
         x.full = 1;
         x.live = p.nchunks;
         if (p.planned) {
@@ -516,7 +518,7 @@ __global__ __launch_bounds__(kWave * kQueriesPerGroup / QPW) void score_shared(S
             x.fills = p.groups * ((rest + x.fill - 1) / x.fill);
         }
         total_items = x.live_items + x.fills;
-        if (t == 0) plan = x;
+        if (HB == 4 && t == 0) plan_sh = x;
     } else {
         total_items = 0;
 #pragma unroll
