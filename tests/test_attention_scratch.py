@@ -1,6 +1,7 @@
-"""The scratch of attend_slots (partial sums between its two launches) belongs
-to one call: calls of other threads on the same stream, and graphs captured on
-one stream and replayed side by side, have their own."""
+"""The scratch of attend_slots (partial sums between the two launches of a call of
+more than 2^18 keys in all) belongs to one call: calls of other threads on the
+same stream, and graphs captured on one stream and replayed side by side, have
+their own."""
 import threading
 
 import pytest
@@ -32,13 +33,13 @@ def test_a_call_between_the_launches_of_another_has_its_own_scratch(monkeypatch)
     def call(name, *args):
         assert name == "v1_decode_attention_slots_ws"
         at, size = args[-3], args[-2]
-        assert at and size == L.lib().v1_decode_attention_slots_workspace(rows, 4, 512)
+        assert at and size == L.lib().v1_decode_attention_slots_workspace(rows, 4, 2048)
         ranges.append((at, at + size))
         if len(ranges) == 1:
             AT.attend_slots(*inputs)
 
-    rows = 8
-    inputs = _inputs(1, rows, 512, "cpu")
+    rows = 136
+    inputs = _inputs(1, rows, 2048, "cpu")
     monkeypatch.setattr(L, "call", call)
     monkeypatch.setattr(L, "require_gpu", lambda *tensors: None)
     monkeypatch.setattr(L, "stream_of", lambda t: 0)
@@ -50,7 +51,8 @@ def test_a_call_between_the_launches_of_another_has_its_own_scratch(monkeypatch)
 
 @pytest.mark.gpu
 def test_threads_on_one_stream():
-    sets = [_inputs(s, rows, keys, "cuda:0") for s, (rows, keys) in enumerate([(8, 2048), (8, 2048), (64, 512), (300, 1000)])]
+    sets = [_inputs(s, rows, keys, "cuda:0") for s, (rows, keys) in enumerate([(136, 2048), (136, 2048), (600, 512), (300, 1000)])]
+    assert all(L.lib().v1_decode_attention_slots_workspace(len(x[0]), 4, x[4].shape[1]) > 0 for x in sets)
     want = [AT.attend_slots(*x) for x in sets]
     torch.cuda.synchronize()
     got, start = [[] for _ in sets], threading.Barrier(len(sets))
@@ -73,7 +75,7 @@ def test_threads_on_one_stream():
 @pytest.mark.gpu
 def test_graphs_captured_on_one_stream_replayed_on_two():
     s = torch.cuda.Stream()
-    sets = [_inputs(s_, 32, 2048, "cuda:0") for s_ in (1, 2)]
+    sets = [_inputs(s_, 136, 2048, "cuda:0") for s_ in (1, 2)]
     want = [AT.attend_slots(*x) for x in sets]
     torch.cuda.synchronize()
     graphs, outs = [], []
