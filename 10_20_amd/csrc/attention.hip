@@ -34,7 +34,8 @@
 // is 20-22 TB/s, which the L2s must give; 1 head 486 -> 190 us), one row 97 ->
 // 15 us, 1024 rows of 128 keys 18 -> 15 us.  One head of at most 96 keys alone
 // is slower than it was, by 0.1-0.5 us up to 1024 rows (4096 rows of 64 keys 23
-// -> 26 us): the prologue's and the join's latency.  Over rows of contiguous
+// -> 26 us): the prologue's and the join's latency.  So are gathered keys of one
+// head per KV head, by 2-10% (512 rows x 1024 keys 39.5 -> 43.3 us).  Over rows of contiguous
 // keys (nothing shared) 822 -> 704 us, HBM's rate.
 //
 // Slot form: keys come straight from the K / V pools of one KV head through
@@ -53,7 +54,7 @@ namespace {
 
 constexpr int kAttnDim = 128;
 constexpr int kMaxGroup = 4;       // heads of a P fragment: 16 rows / (3 parts, one unused)
-constexpr int kMaxScores = 12288;  // keys x heads that a call may have
+constexpr int kMaxScores = 12288;  // keys x heads that a call may have (the entries' limit, not these kernels')
 constexpr int kTile = 32;          // keys per step of a wave
 constexpr int kMaxWaves = 16;      // waves of a work-group
 constexpr int kXcds = 8;

@@ -15,11 +15,12 @@
 // u_d = fl(x_d / m), c_d the FP8 key and s its scale.  Center means add the 8
 // members in order, times 1/8.
 //
-// Two forms: per-kernel drop-ins with the reference's launch shapes, and two
+// Two forms: per-kernel drop-ins with the reference's launch shapes, and three
 // launches that build a batch of buckets (thread = position in the order):
-// build_top_kernel takes a bucket through the groups of 1024 and 512 with the
-// tokens' FP8 keys in registers, build_quarter_kernel a quarter of it through
-// the groups of 256 to 16 with their unit vectors there.  An argmin winner
+// build_top_kernel takes a bucket through the groups of 1024 and, launched
+// again, of 512 with the tokens' FP8 keys in registers, build_quarter_kernel a
+// quarter of it through the groups of 256 to 16 with their unit vectors there
+// (and build_write_kernel writes outputs that lie over the pool).  An argmin winner
 // stages its vector in LDS, each group is sorted by a bitonic network over its
 // unique (score, -position) words, and members move through LDS or lane
 // permutes.
@@ -30,9 +31,10 @@
 // lower levels keep the components (128 registers a token, which is why a
 // work-group is a quarter: three share a CU) and a term of a dot costs its
 // product and its sum; the anchor's components come by DPP row broadcast as
-// an operand of the product, from 8 registers a lane.  2048 buckets take
-// 161 + 131 + 459 us (one launch with every component made anew for every dot
-// 1266), four 24 + 14 + 25 us (155); the vector units issue 94-96% of the time.
+// an operand of the product, from 8 registers a lane.  2048 buckets take 695-712
+// us (under the profiler, which slows them, 164 + 131 + 464; one launch with
+// every component made anew for every dot 1266), four 63.6 us (24 + 14 + 26;
+// 155); the vector units issue 94-96% of the time.
 #include <type_traits>
 
 #include "common.h"

@@ -1,7 +1,7 @@
 """Batched index build: the producer chain of
 sglang/srt/layers/attention/v1_deepseek/runtime.py:171-216 (initialize,
 seven levels of _dots / _anchor / _sort, assemble) for many 1024-token
-buckets in one launch, one work-group per bucket.
+buckets in one call (three launches for the whole batch).
 
 build_buckets(pool, tables, starts) -> (perm, tmp, mapping, centers):
   pool     uint8 [pages, 8448] native pages (128 FP8 bytes per token, then 64
@@ -14,7 +14,10 @@ build_buckets(pool, tables, starts) -> (perm, tmp, mapping, centers):
   centers  uint8 [buckets, 2, 8448]: 128 FP8 centers (means of 8 members)
            with their power-of-two scales
 Results equal the chain of the per-kernel drop-ins (kernels.initialize,
-fused_grouping._dots/_anchor/_sort, kernels.assemble) bit for bit.
+fused_grouping._dots/_anchor/_sort, kernels.assemble) bit for bit.  `out` may
+hold tensors over a bucket's own source pages (tmp = the pool sorts its pages
+where they lie), not over another bucket's; with tmp over the pool, perm and
+mapping lie apart from it and from each other.
 """
 import torch
 

@@ -22,7 +22,7 @@ PCG64, resident in HBM before timing starts).  Workloads (--config):
                score -> mask -> Top-2048 -> raw/logical/physical map -> gather (the
                full-scoring chain over every context key timed beside it)
   6            index build: every 1024-token bucket of a 2M-token FP8 pool (2048 buckets)
-               -> member order, reordered pages and FP8 centers, one launch
+               -> member order, reordered pages and FP8 centers, one call
   8            attention consumer: 4096 queries x 4 heads of one KV head, 2048 gathered bf16
                K/V slots each (1M-slot pool) -> decode attention
   10           context timings, microseconds per call under HIP graph replay: _sort of one
@@ -61,10 +61,10 @@ TRAFFIC = {
     4: (ROOT / "profiles" / "prefill_chunk_4096x32k.md",
         {"score": ("score_prep", "score_shared", "score_exact"), "topk": ("transform_rows",), "gather": ("gather_rows16",)}),
     3: (ROOT / "profiles" / "slot_gather_1024x2048.md", {"gather": ("gather_rows16",)}),
-    6: (ROOT / "profiles" / "index_build_2048x1024.md", {"build": ("build_buckets_kernel",)}),
+    6: (ROOT / "profiles" / "index_build_2048x1024.md", {"build": ("build_top_kernel", "build_quarter_kernel")}),
     2: (ROOT / "profiles" / "page_management_4096req.md",
         {"insert": ("pb_init", "pb_hash", "pb_classify", "pb_slow_live", "pb_slow", "pb_allocate", "pb_table",
-                    "pb_publish", "pb_commit")}),
+                    "pb_publish")}),
 }
 
 

@@ -1,7 +1,7 @@
 """Index-build producer on the GPU against the oracle: the per-kernel drop-ins
 (kernels.initialize / assemble, fused_grouping._dots / _anchor / _sort) with
 the reference's launch shapes, their chain as runtime.py:171-216 runs it, and
-the batched one-launch build (indexbuild.build_buckets), bit for bit."""
+the batched build (indexbuild.build_buckets), bit for bit."""
 import importlib
 import sys
 from pathlib import Path
