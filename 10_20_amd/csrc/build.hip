@@ -766,7 +766,7 @@ extern "C" int v1_build_buckets(const void* pool, int64_t pool_pages, const int3
     // Outputs over a bucket's own pages are allowed (all of the bucket is read
     // before any of them is written); quarters that read and write side by side
     // are for outputs elsewhere.  The order between the launches lies in tmp, or
-    // in perm and mapping where tmp is over the pool.
+    // where tmp is over the pool in centers, or else in perm and mapping.
     const int64_t pool_bytes = pool_pages * V1_PAGE_BYTES, order_bytes = (int64_t)buckets * kTokens * 4;
     auto meet = [](const void* a, int64_t na, const void* b, int64_t nb) {
         const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
@@ -774,13 +774,17 @@ extern "C" int v1_build_buckets(const void* pool, int64_t pool_pages, const int3
     };
     const bool tmp_meets = meet(pool, pool_bytes, tmp, (int64_t)buckets * 16 * V1_PAGE_BYTES);
     const bool order_meets = meet(pool, pool_bytes, perm, order_bytes) || meet(pool, pool_bytes, mapping, order_bytes);
-    const bool in_place = tmp_meets || order_meets ||
-                          meet(pool, pool_bytes, centers, (int64_t)buckets * 2 * V1_PAGE_BYTES);
-    V1_REQUIRE(!tmp_meets || !(order_meets || meet(perm, order_bytes, mapping, order_bytes)),
-               "build_buckets: with tmp over the pool, perm and mapping must be apart from it and from each other");
+    const bool centers_meet = meet(pool, pool_bytes, centers, (int64_t)buckets * 2 * V1_PAGE_BYTES);
+    const bool in_place = tmp_meets || order_meets || centers_meet;
+    V1_REQUIRE(!tmp_meets || !centers_meet || !(order_meets || meet(perm, order_bytes, mapping, order_bytes)),
+               "build_buckets: with tmp and centers over the pool, perm and mapping must be apart from it and from "
+               "each other");
     Carry carry{perm, reinterpret_cast<float*>(mapping), kTokens, kQuarter};
     if (!tmp_meets) {
         carry = Carry{static_cast<int32_t*>(tmp), static_cast<float*>(tmp) + kQuarter, 16 * kPageWords, 4 * kPageWords};
+    } else if (!centers_meet) {
+        static_assert(2 * kTokens <= 2 * kPageWords, "order and divisors of a bucket in its two center pages");
+        carry = Carry{static_cast<int32_t*>(centers), static_cast<float*>(centers) + kTokens, 2 * kPageWords, kQuarter};
     }
     const uint8_t* const from = static_cast<const uint8_t*>(pool);
     uint8_t* const pages = static_cast<uint8_t*>(tmp);

@@ -16,8 +16,8 @@ build_buckets(pool, tables, starts) -> (perm, tmp, mapping, centers):
 Results equal the chain of the per-kernel drop-ins (kernels.initialize,
 fused_grouping._dots/_anchor/_sort, kernels.assemble) bit for bit.  `out` may
 hold tensors over a bucket's own source pages (tmp = the pool sorts its pages
-where they lie), not over another bucket's; with tmp over the pool, perm and
-mapping lie apart from it and from each other.
+where they lie), not over another bucket's; with both tmp and centers over
+the pool, perm and mapping lie apart from it and from each other.
 """
 import torch
 

@@ -360,8 +360,8 @@ int v1_build_assemble(const void* K, const float* KS, const int32_t* table, cons
  * results to the chain of the entry points above.  Table entries outside
  * [0, pool_pages) read page 0.  A bucket's outputs may lie over its own source
  * pages (all of the bucket is read before any of them is written), not over
- * another bucket's; with tmp over the pool, perm and mapping must lie apart
- * from the pool and from each other (they hold the order meanwhile). */
+ * another bucket's; with both tmp and centers over the pool, perm and mapping
+ * must lie apart from it and from each other (they hold the order meanwhile). */
 int v1_build_buckets(const void* pool, int64_t pool_pages, const int32_t* tables, const int32_t* starts,
                      int32_t buckets, int32_t* perm, void* tmp, int32_t* mapping, void* centers, void* stream);
 

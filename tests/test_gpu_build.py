@@ -219,8 +219,8 @@ def test_build_buckets_scales(mods, factors):
 @pytest.mark.parametrize("buckets", [1, 5])
 def test_build_buckets_in_place(mods, buckets):
     """tmp over the buckets' own source pages (each bucket's pages sorted where
-    they lie), centers over the first two of them, mapping over perm: the bytes
-    of a call with outputs of their own."""
+    they lie), other outputs over them too, mapping over perm: the bytes of a
+    call with outputs of their own, wherever the order lies meanwhile."""
     _, _, IB = mods
     g = np.random.default_rng(buckets)
     pool = T(np.concatenate([_pool(40 + i) for i in range(buckets)])[:16 * buckets])
@@ -252,6 +252,15 @@ def test_build_buckets_in_place(mods, buckets):
     p, o = pool.clone(), outs()
     o[1] = p.view(buckets, 16, 8448)
     o[0] = o[2].view(buckets, 1024)
-    with pytest.raises(ValueError, match="apart"):
-        IB.build_buckets(p, tables, starts, out=o)
-    assert torch.equal(p, pool)
+    check(IB.build_buckets(p, tables, starts, out=o), skip=(0,))
+    if buckets == 1:  # tmp over the source pages, centers over others of the pool: the order lies in perm and mapping
+        p = torch.cat([pool[:2].clone(), pool, pool[:2].clone()])
+        o = outs()
+        o[1], o[3] = p[2:18][None], p[18:20][None]
+        check(IB.build_buckets(p, tables + 2, starts, out=o))
+        p = torch.cat([pool, pool[:2].clone()])
+        o[1], o[3] = p[:16][None], p[16:18][None]
+        o[0] = o[2].view(buckets, 1024)
+        with pytest.raises(ValueError, match="apart"):
+            IB.build_buckets(p, tables, starts, out=o)
+        assert torch.equal(p[:16], pool)
